@@ -64,14 +64,14 @@ def main():
     c1 = round_bits(c, 32)
     c2 = rn(c - c1)
     c3 = rn(c - c1 - c2)
-    w("PP_CR_TAB double pp_cr_exp_c[4] = {%s, %s, %s, %s};  // 128/ln2, ln2/128 = C1 + C2 + C3"
+    w("PP_CR_CST double pp_cr_exp_c[4] = {%s, %s, %s, %s};  // 128/ln2, ln2/128 = C1 + C2 + C3"
       % (hexs(rn(128 / ln2)), hexs(c1), hexs(c2), hexs(c3)))
     w("PP_CR_TAB double pp_cr_exp_t[256] = {  // 2^(j/128): hi, lo")
     for j in range(128):
         hi, lo = dd(mp.mpf(2) ** (mp.mpf(j) / 128))
         w("    %s, %s," % (hexs(hi), hexs(lo)))
     w("};")
-    w("PP_CR_TAB double pp_cr_exp_p[8] = {  // 1/k!, k = 0..7")
+    w("PP_CR_CST double pp_cr_exp_p[8] = {  // 1/k!, k = 0..7")
     w("    " + ", ".join(hexs(rn(1 / mp.factorial(k))) for k in range(8)) + ",")
     w("};")
     w("PP_CR_TAB double pp_cr_exp_pdd[28] = {  // 1/k!, k = 0..13: hi, lo")
@@ -83,7 +83,7 @@ def main():
     ln2hi = round_bits(ln2, 42)
     ln2lo = rn(ln2 - ln2hi)
     ln2lo2 = rn(ln2 - ln2hi - ln2lo)
-    w("PP_CR_TAB double pp_cr_ln2[3] = {%s, %s, %s};  // ln2 = hi (42 bits) + lo + lo2"
+    w("PP_CR_CST double pp_cr_ln2[3] = {%s, %s, %s};  // ln2 = hi (42 bits) + lo + lo2"
       % (hexs(ln2hi), hexs(ln2lo), hexs(ln2lo2)))
     inv, Lhi, Llo = [], [], []
     umax = mp.mpf(0)
@@ -111,7 +111,7 @@ def main():
     for j in range(96):
         w("    %s, %s," % (hexs(Lhi[j]), hexs(Llo[j])))
     w("};")
-    w("PP_CR_TAB double pp_cr_log_p[16] = {  // (-1)^(k+1)/k, k = 1..16")
+    w("PP_CR_CST double pp_cr_log_p[16] = {  // (-1)^(k+1)/k, k = 1..16")
     w("    " + ", ".join(hexs(rn(mp.mpf((-1) ** (k + 1)) / k)) for k in range(1, 17)) + ",")
     w("};")
     w("PP_CR_TAB double pp_cr_log_pdd[36] = {  // (-1)^(k+1)/k, k = 1..18: hi, lo")

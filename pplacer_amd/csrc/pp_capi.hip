@@ -599,9 +599,18 @@ size_t stage2_lds(const pp_ctx *c, int bd, size_t taken, int spl, int stream_cap
   const MWLayout<Real, R, STRICT> lay(c->model.n_cats > 0 ? c->model.n_cats : 1, c->model.n_sl(), cap, spl == 0);
   return lay.align(lay.align(lay.bytes()) + taken) + (spl ? MWProducts<Real, R * 4>::bytes(cap) : 0);
 }
-size_t stage2_lds_fp64(const pp_ctx *c, int bd, size_t taken, int spl, int stream_cap) {
-  return c->model.R == 4 ? stage2_lds<double, 4, true>(c, bd, taken, spl, stream_cap)
-                         : stage2_lds<double, 1, true>(c, bd, taken, spl, stream_cap);
+// LDS by which a masked length is classed and accepted: a fixed account of the
+// FP64 workgroup (header and tables, 16 bytes of log sum and 4 or 8 of list a
+// site, 1 KB, the pitch kernel's flags, products), never less than the layout
+// takes, so that neither the class limits nor the longest query the GPU path
+// takes move when the layout does.
+size_t accept_lds(const pp_ctx *c, int bd, size_t taken, int spl, int stream_cap) {
+  const size_t cap = spl == 0 ? stream_cap : (bd - 64) * spl, R = c->model.R, n_sl = c->model.n_sl();
+  const size_t n_tsl = c->model.n_cats > 0 ? c->model.n_cats : 1;
+  const auto align = [](size_t v) { return (v + 15) & ~size_t(15); };
+  const size_t base = 2144 + 8 * n_tsl * 32 * R * 4 + 2 * 8 * n_sl * 16 + 8 * 3 * n_sl * 4 + 16 * cap + 1024;
+  const size_t products = R == 4 ? MWProducts<double, 16>::bytes((int)cap) : MWProducts<double, 4>::bytes((int)cap);
+  return align(align(base + 4 * cap * (spl ? 1 : 2)) + taken) + (spl ? products : 0);
 }
 
 // Whether the FP32 form runs stage 2 in FP32.  The 20-state engine evaluates
@@ -622,23 +631,23 @@ int register_limit(const pp_ctx *c) {
   for (int b = 0; b < kLongBucket; b++) {
     const int spl = spl_for(true, b), bd = block_for(b, spl);
     if (bd > 1024) break;
-    if (stage2_lds_fp64(c, bd, taken_bytes(c->E), spl, 0) > c->max_lds) break;
+    if (accept_lds(c, bd, taken_bytes(c->E), spl, 0) > c->max_lds) break;
     m = 64 * (b + 1);
   }
   return m;
 }
 
 // Longest masked length the GPU path places: N for 20 states (pair state in
-// global scratch); for 4 states the streaming form's, whose LDS holds 16
-// bytes per masked site (log, column, pendant row) besides the header and
-// flags, so about 9,000 sites in the 160 KB of a gfx950 workgroup.  Longer
+// global scratch); for 4 states the streaming form's, with 24 bytes of
+// LDS counted per masked site besides the header and flags, so about 6,500
+// sites in the 160 KB of a gfx950 workgroup.  Longer
 // queries get PP_Q_RANK_EXHAUSTED ("query too long for the GPU path").
 int max_masked_sites(const pp_ctx *c) {
   if (c->model.S == 20) return c->N;
   int lo = 0, hi = c->N;
   while (lo < hi) {  // largest cap whose streaming workgroup fits
     const int mid = lo + (hi - lo + 1) / 2;
-    if (stage2_lds_fp64(c, 1024, taken_bytes(c->E), 0, mid) <= c->max_lds) lo = mid;
+    if (accept_lds(c, 1024, taken_bytes(c->E), 0, mid) <= c->max_lds) lo = mid;
     else hi = mid - 1;
   }
   return std::max(lo, std::min(register_limit(c), c->N));
@@ -2212,14 +2221,14 @@ int pp_ten_bounded_logdot(const double *x, const double *y, int first, int last,
 // Test hook, not part of the drop-in ABI: the FP64 engine's wave-parallel
 // sequential sum (wave_sequential_sum) over x[0..n), copied into LDS, beside
 // the one-lane chain.  out[0] = the wave's sum, out[1] = the chain's, out[2] =
-// the number of events (-1 where the wave fell back to the chain).
+// the number of blocks added from the true sum (-1 where the chain ran).
 static __global__ void seqsum_test_kernel(const double *x, int n, double *out) {
-  extern __shared__ __align__(16) double sm[];
-  double *v = sm, *acc = sm + n, *ev = sm + 2 * (size_t)n;
-  for (int i = threadIdx.x; i < n; i += blockDim.x) v[i] = x[i];
+  extern __shared__ __align__(16) double v[];
+  const int n_pad = (n + 63) & ~63;
+  for (int i = threadIdx.x; i < n_pad; i += blockDim.x) v[i] = i < n ? x[i] : 0.0;
   __syncthreads();
   int n_events = 0;
-  const double s = wave_sequential_sum(v, n, acc, ev, &n_events);
+  const double s = wave_sequential_sum(v, n, &n_events);
   const double c = threadIdx.x == 0 ? ordered_sum(v, n) : 0.0;
   if (threadIdx.x == 0) {
     out[0] = s;
@@ -2233,7 +2242,7 @@ int pp_test_sequential_sum(const double *x, int n, double *out) {
   int dev = 0, max_lds = 65536;
   HIPCHECK(hipGetDevice(&dev));
   if (hipDeviceGetAttribute(&max_lds, hipDeviceAttributeMaxSharedMemoryPerBlock, dev) != hipSuccess) max_lds = 65536;
-  const size_t lds = sizeof(double) * (2 * (size_t)n + 2 * kSeqSumEvents);
+  const size_t lds = sizeof(double) * (((size_t)n + 63) & ~(size_t)63);
   CHECK(lds <= (size_t)max_lds, PP_EINVAL, "n exceeds one workgroup's LDS");
   Scratch s;
   double *dx = s.up(x, std::max(n, 1)), *dout = s.up<double>(nullptr, 3);

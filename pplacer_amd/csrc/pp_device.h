@@ -49,6 +49,20 @@ __device__ __forceinline__ double readlane_f64(double v, int l) {
   return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
 }
 
+// A condition on wave-uniform values (every lane of the wave active) as a
+// scalar one, so that a branch on it is a scalar branch and what it decides
+// stays known to be uniform.
+__device__ __forceinline__ bool wave_true(bool c) { return __builtin_amdgcn_ballot_w64(c) != 0; }
+
+// A wave-uniform double moved to scalar registers: for control values that
+// live long between uses, which then cost no vector register.
+__device__ __forceinline__ double scalar(double v) {
+  const unsigned long long b = (unsigned long long)__double_as_longlong(v);
+  const unsigned lo = (unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)b);
+  const unsigned hi = (unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)(b >> 32));
+  return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
+}
+
 // v from the lane the DPP control CTRL selects (every lane of the wave active)
 template <int CTRL>
 __device__ __forceinline__ double dpp_f64(double v) {

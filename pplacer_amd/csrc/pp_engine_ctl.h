@@ -56,11 +56,13 @@ __device__ __forceinline__ double qng_rescale_error(double err, double result_ab
 // the 21-point Gauss-Kronrod rule checked against the 10-point Gauss rule,
 // then Patterson's 43- and 87-point extensions reusing every evaluation.  f is
 // evaluated at one call site, at the centre and then at the +/- pairs of the
-// tables in order; f(x, err) sets err to abandon the rule.
+// tables in order; f(x, err) sets err to abandon the rule.  With `centre_only`
+// the result is f at the centre, no integral.
 template <class F>
 __device__ __forceinline__ int qng(F &&f, double a, double b, double epsrel, LaneStore &st,
-                                   double *result) {
+                                   double *result, bool centre_only = false) {
   *result = 0;
+  if (centre_only) epsrel = 1.;
   if (epsrel < 50 * DBL_EPSILON || epsrel < 0.5e-28) return QNG_EBADTOL;
   const double half_length = 0.5 * (b - a), abs_half_length = fabs(half_length);
   const double center = 0.5 * (b + a);
@@ -82,6 +84,7 @@ __device__ __forceinline__ int qng(F &&f, double a, double b, double epsrel, Lan
       int err = 0;
       const double v = f(x, err);
       if (err) return QNG_ABORT;
+      if (centre_only) { *result = v; return QNG_OK; }
       st.put(j, v);
     }
     const double fc = st.get(0);
@@ -132,7 +135,7 @@ __device__ __forceinline__ int qng(F &&f, double a, double b, double epsrel, Lan
     const double result_kronrod = res * half_length;
     const double err = qng_rescale_error(diff * half_length, resabs, resasc);
     *result = result_kronrod;
-    if (err < 0. || err < epsrel * fabs(result_kronrod)) return QNG_OK;
+    if (wave_true(err < 0. || err < epsrel * fabs(result_kronrod))) return QNG_OK;
     prev = res;
   }
   return QNG_ETOL;  // "failed to reach tolerance with highest-order rule"
@@ -166,11 +169,11 @@ struct ThreeTaxControl {
   // ---- Minimization.brent with the GSL Brent minimiser ---------------------
   // kind 0: pendant (three_tax.ml:38-39), 1: distal (three_tax.ml:41-45),
   // 2: find_upper_limit's |target - (log_like + log prior)| over the pendant
-  // length (three_tax.ml:142-149)
+  // length (three_tax.ml:142-149), -1: one likelihood at the current state
   __device__ __forceinline__ double fprobe(int kind, double v, int &err) {
     if (kind == 1) {
       const double prox = (dist_bl + prox_bl) - v;
-      if (!(prox >= 0.)) err = ST_ASSERT;
+      if (wave_true(!(prox >= 0.))) err = ST_ASSERT;
       dist_bl = v;
       prox_bl = prox;
     } else {
@@ -182,78 +185,128 @@ struct ThreeTaxControl {
     return x == INFINITY ? 100000.0 : x;
   }
 
+  // One loop around one probe: `phase` says what the probe at x was for.  A
+  // probe (transition tables, command, log sum) is then one piece of code
+  // instead of one per place that asks for a likelihood, and the control's
+  // values stay in registers across it: the 4-state FP64 baseball kernel went
+  // from 50 to 18 KB of code.  Values are wave-uniform, and branches on them
+  // go through wave_true, so they are scalar branches.
   __device__ __forceinline__ int brent(int kind, double raw_start, double left, double right, double tol,
                        int max_iters, double *result) {
-    int err = 0;
-    if (left >= raw_start || raw_start >= right) return ST_INVALID_START;
-    const double righty = fprobe(kind, right, err);  // (f left, f right) evaluates right first
-    if (err) return err;
-    const double prox_r = prox_bl;
-    const double lefty = fprobe(kind, left, err);
-    if (err) return err;
-    const double prox_l = prox_bl;
-    const double smaller = lefty < righty ? left : right;
-    const double miny = lefty <= righty ? lefty : righty;  // Stdlib.min
-    double prev = raw_start, pv, prox_p;
-    for (int iter = 1;; iter++) {
-      pv = fprobe(kind, prev, err);
-      if (err) return err;
-      prox_p = prox_bl;
-      if (pv < miny) break;
-      if (fabs(prev - smaller) < tol) { *result = smaller; return ST_OK; }  // FoundMin
-      if (iter > max_iters) return ST_FIND_START;
-      prev = (prev + smaller) / 2.;
-    }
-    // gsl_min_fminimizer_set evaluates f(lower), f(upper), f(start) again.  A
-    // pendant probe moves only the pendant length, so those are the values
-    // just computed, and the state is already at start.  A distal probe also
-    // moves the proximal length to (dist + prox) - v, whose rounding drifts
-    // from probe to probe: the three moves are replayed in the set's order,
-    // with their assertion, and a value is reused only where the proximal
-    // length comes out bit-identical to the one it was computed at.
-    double x_lower = left, x_upper = right, x_min = prev;
-    double f_lower = lefty, f_upper = righty, f_min = pv;
-    // (scalar selects and one probe site: no addressable locals in the loop)
-#pragma nounroll
-    for (int k = 0; k < 3; k++) {
-      const double x = k == 0 ? left : k == 1 ? right : prev;
-      double f = k == 0 ? f_lower : k == 1 ? f_upper : f_min;
-      if (kind == 1) {
-        const double prox = (dist_bl + prox_bl) - x;
-        if (prox == (k == 0 ? prox_l : k == 1 ? prox_r : prox_p)) {
-          dist_bl = x;
-          prox_bl = prox;
-          n_calls++;  // the reference's call, answered from the value at hand
-        } else {
-          f = fprobe(kind, x, err);
-          if (err) return err;
-        }
-      } else {
-        n_calls++;
-      }
-      if (!isfinite(f)) return ST_GSL_BADFUNC;
-      if (k == 0) f_lower = f;
-      else if (k == 1) f_upper = f;
-      else f_min = f;
-    }
-    if (x_lower > x_upper || x_min >= x_upper || x_min <= x_lower) return ST_GSL;
-    if (f_min >= f_lower || f_min >= f_upper) return ST_GSL;
+    enum { P_RIGHT, P_LEFT, P_START, P_SET, P_FIRST, P_STEP, P_ONLY };
+    if (kind >= 0 && wave_true(left >= raw_start || raw_start >= right)) return ST_INVALID_START;
     const double golden = 0.3819660;
-    double v = x_lower + golden * (x_upper - x_lower), w_ = v;
-    double sd = 0., se = 0.;
-    double f_v = fprobe(kind, v, err);
-    if (err) return err;
-    if (!isfinite(f_v)) return ST_GSL_BADFUNC;
-    double f_w = f_v;
-    for (int step = 1;; step++) {
-      if (step > max_iters) return ST_MAXITER;
+    // count: start finder's iteration, set's move, then Brent's step
+    int err = 0, phase = kind < 0 ? P_ONLY : P_RIGHT, count = 1;
+    double x = kind < 0 ? raw_start : right;  // (f left, f right) evaluates right first
+    double x_lower = left, x_upper = right, x_min = raw_start;
+    double f_lower = 0., f_upper = 0., f_min = 0.;
+    // Brent's older points; until then v, w_ and f_v hold the proximal lengths
+    // at which f left, f right and f start were computed, sd the smaller end
+    // and se its value
+    double v = 0., w_ = 0., f_v = 0., f_w = 0., sd = 0., se = 0.;
+#pragma unroll 1
+    for (;;) {
+      double f = fprobe(kind, x, err);
+      if (err || phase == P_ONLY) return err;
+      if (phase < P_SET) {
+        if (phase == P_RIGHT) {
+          f_upper = f;
+          w_ = prox_bl;
+          x = left;
+          phase = P_LEFT;
+          continue;
+        }
+        if (phase == P_LEFT) {
+          f_lower = f;
+          v = prox_bl;
+          sd = f_lower < f_upper ? left : right;
+          se = f_lower <= f_upper ? f_lower : f_upper;  // Stdlib.min
+          x = x_min;
+          phase = P_START;
+          continue;
+        }
+        f_min = f;
+        f_v = prox_bl;
+        if (wave_true(!(f < se))) {
+          if (wave_true(fabs(x_min - sd) < tol)) { *result = sd; return ST_OK; }  // FoundMin
+          if (count > max_iters) return ST_FIND_START;
+          count++;
+          x = x_min = (x_min + sd) / 2.;
+          continue;
+        }
+        count = 0;
+      }
+      if (phase <= P_SET) {
+        // gsl_min_fminimizer_set evaluates f(lower), f(upper), f(start) again.  A
+        // pendant probe moves only the pendant length, so those are the values
+        // just computed, and the state is already at start.  A distal probe also
+        // moves the proximal length to (dist + prox) - v, whose rounding drifts
+        // from probe to probe: the three moves are replayed in the set's order,
+        // with their assertion, and a value is reused only where the proximal
+        // length comes out bit-identical to the one it was computed at.
+        bool probed = phase == P_SET, again = false;
+#pragma unroll 1
+        for (; count < 3; count++) {
+          const double at = count == 0 ? x_lower : count == 1 ? x_upper : x_min;
+          if (!probed) {
+            f = count == 0 ? f_lower : count == 1 ? f_upper : f_min;
+            if (kind == 1) {
+              const double prox = (dist_bl + prox_bl) - at;
+              if (wave_true(!(prox == (count == 0 ? v : count == 1 ? w_ : f_v)))) {
+                x = at;
+                again = true;
+                break;
+              }
+              dist_bl = at;
+              prox_bl = prox;
+            }
+            n_calls++;  // the reference's call, answered from the value at hand
+          }
+          probed = false;
+          if (wave_true(!isfinite(f))) return ST_GSL_BADFUNC;
+          if (count == 0) f_lower = f;
+          else if (count == 1) f_upper = f;
+          else f_min = f;
+        }
+        phase = P_SET;
+        if (again) continue;
+        if (wave_true(x_lower > x_upper || x_min >= x_upper || x_min <= x_lower)) return ST_GSL;
+        if (wave_true(f_min >= f_lower || f_min >= f_upper)) return ST_GSL;
+        x = v = w_ = x_lower + golden * (x_upper - x_lower);
+        sd = se = 0.;
+        count = 0;
+        phase = P_FIRST;
+        continue;
+      }
+      if (wave_true(!isfinite(f))) return ST_GSL_BADFUNC;
+      if (phase == P_FIRST) {
+        f_v = f_w = f;
+        phase = P_STEP;
+      } else {
+        const double u = x, f_u = f, z = x_min, f_z = f_min;
+        const bool left_of = u < z;
+        if (wave_true(f_u <= f_z)) {
+          if (left_of) { x_upper = z; f_upper = f_z; }
+          else { x_lower = z; f_lower = f_z; }
+          v = w_; f_v = f_w; w_ = z; f_w = f_z;
+          x_min = u; f_min = f_u;
+        } else {
+          if (left_of) { x_lower = u; f_lower = f_u; }
+          else { x_upper = u; f_upper = f_u; }
+          if (f_u <= f_w || w_ == z) { v = w_; f_v = f_w; w_ = u; f_w = f_u; }
+          else if (f_u <= f_v || v == z || v == w_) { v = u; f_v = f_u; }
+        }
+        if (wave_true(x_upper - x_lower < tol)) { *result = x_min; return ST_OK; }
+      }
+      if (++count > max_iters) return ST_MAXITER;
       const double x_left = x_lower, x_right = x_upper, z = x_min, f_z = f_min;
       double d = se, e = sd, u;
       const double w_lower = z - x_left, w_upper = x_right - z;
       const double tl = 1.4901161193847656e-08 * fabs(z);
       double p = 0, q = 0, r = 0;
       const double midpoint = 0.5 * (x_left + x_right);
-      if (fabs(e) > tl) {
+      if (wave_true(fabs(e) > tl)) {
         r = (z - w_) * (f_z - f_v);
         q = (z - v) * (f_z - f_w);
         p = (z - v) * q - (z - w_) * r;
@@ -262,7 +315,7 @@ struct ThreeTaxControl {
         r = e;
         e = d;
       }
-      if (fabs(p) < fabs(0.5 * q * r) && p < q * w_lower && p < q * w_upper) {
+      if (wave_true(fabs(p) < fabs(0.5 * q * r) && p < q * w_lower && p < q * w_upper)) {
         const double t2 = 2 * tl;
         d = p / q;
         u = z + d;
@@ -275,46 +328,39 @@ struct ThreeTaxControl {
       else u = z + ((d > 0) ? tl : -tl);
       se = e;
       sd = d;
-      const double f_u = fprobe(kind, u, err);
-      if (err) return err;
-      if (!isfinite(f_u)) return ST_GSL_BADFUNC;
-      if (f_u <= f_z) {
-        if (u < z) { x_upper = z; f_upper = f_z; }
-        else { x_lower = z; f_lower = f_z; }
-        v = w_; f_v = f_w; w_ = z; f_w = f_z;
-        x_min = u; f_min = f_u;
-      } else {
-        if (u < z) { x_lower = u; f_lower = f_u; }
-        else { x_upper = u; f_upper = f_u; }
-        if (f_u <= f_w || w_ == z) { v = w_; f_v = f_w; w_ = u; f_w = f_u; }
-        else if (f_u <= f_v || v == z || v == w_) { v = u; f_v = f_u; }
-      }
-      if (x_upper - x_lower < tol) { *result = x_min; return ST_OK; }
+      x = u;
     }
   }
 
-  // three_tax.ml:48-58
-  __device__ __forceinline__ int optimize_something(int kind, double tol, double start_v, double min_v,
-                                    double max_v, double *res) {
-    if (min_v == max_v) { *res = start_v; return ST_OK; }
-    return brent(kind, start_v, min_v, max_v, tol, 100, res);
-  }
-
-  // three_tax.ml:70-83
+  // three_tax.ml:70-83, each turn optimize_something (three_tax.ml:48-58) of
+  // the pendant (kind 0), then of the distal length (kind 1).  If no turn had
+  // anything to search, one probe (kind -1) gives the likelihood.
   __device__ __forceinline__ int optimize(double tol, double max_pend, int max_iter) {
-    double prev_pend = pend_bl, prev_dist = dist_bl;
-    for (int step = 1;; step++) {
-      if (step > max_iter) return ST_MAXITER;
-      double cp, cd;
-      int st = optimize_something(0, tol, pend_bl, 1e-8, max_pend, &cp);
-      if (st) return st;
-      st = optimize_something(1, tol, dist_bl, 0., dist_bl + prox_bl, &cd);
-      if (st) return st;
-      if (fabs(prev_pend - cp) > tol || fabs(prev_dist - cd) > tol) {
+    double prev_pend = scalar(pend_bl), prev_dist = scalar(dist_bl), cp = 0.;
+#pragma unroll 1
+    for (int step = 1, kind = 0;;) {
+      if (kind == 0 && step > max_iter) return ST_MAXITER;
+      const double start = kind == 1 ? dist_bl : pend_bl;
+      const double lo = kind ? 0. : 1e-8, hi = kind ? dist_bl + prox_bl : max_pend;
+      double at = start;
+      if (kind < 0 || wave_true(lo != hi)) {
+        const int st = brent(kind, start, lo, hi, tol, 100, &at);
+        if (st) return st;
+      }
+      if (kind < 0) return ST_OK;
+      if (kind == 0) {
+        cp = scalar(at);
+        kind = 1;
+        continue;
+      }
+      kind = 0;
+      step++;
+      if (wave_true(fabs(prev_pend - cp) > tol || fabs(prev_dist - at) > tol)) {
         prev_pend = cp;
-        prev_dist = cd;
+        prev_dist = scalar(at);
       } else {
-        return ST_OK;
+        if (have_last) return ST_OK;
+        kind = -1;
       }
     }
   }
@@ -332,10 +378,11 @@ struct ThreeTaxControl {
   // Three_tax.get_results (three_tax.ml:85) at the last probe.
   __device__ __forceinline__ int safe_optimize(double tol, double max_pend, double start_pend, double cut_bl,
                                double *ll, double *pend, double *dist) {
+#pragma unroll 1
     for (int attempt = 0; attempt < 2; attempt++) {
       const int st = optimize(tol, max_pend, 200);
       if (st == ST_OK || st == ST_MAXITER) {
-        *ll = have_last ? last_ll : self().log_like();
+        *ll = last_ll;  // (ExceededMaxIter only after probes)
         *pend = pend_bl;
         *dist = dist_bl;
         return st;
@@ -347,35 +394,35 @@ struct ThreeTaxControl {
   }
 
   // ---- posterior probabilities --------------------------------------------
-  // three_tax.ml:121-163 (the prior is never 0 at the ML pendant length for an
-  // exponential prior short of exp underflow, handled as the reference does)
-  __device__ __forceinline__ int find_upper_limit(double max_pend, double orig_ll, double *limit) {
-    const double orig_pend_bl = pend_bl;
-    if (prior(orig_pend_bl) == 0.) {
-      double curr = orig_pend_bl;
-#pragma unroll 1
-      for (;;) {
-        const double next = curr / 2.;
-        if (prior(next) > exp(-10.)) { *limit = curr; return ST_OK; }
-        curr = next;
-      }
-    }
-    up_target = -10. + orig_ll + log(prior(orig_pend_bl));
-    const double start = orig_pend_bl + (max_pend - orig_pend_bl) / 2.;
-    const int st = brent(2, start, orig_pend_bl, max_pend, 0.02, 10, limit);
-    if (st == ST_GSL) { *limit = max_pend; return ST_OK; }  // Gsl_exn EINVAL
-    return st;
-  }
-
   // three_tax.ml:169-215 at the current state: *marg = base_ll +
   // log(cut_bl^-1 \int_0^cut \int_0^upper exp(ll - base_ll) prior(pend)), the
   // inner range halved on every QNG tolerance failure (at most 10 times).
   __device__ __forceinline__ int calc_marg_prob(double rel_err, double max_pend, double *marg) {
-    const double base_ll = self().log_like();
-    const double cut_bl = dist_bl + prox_bl;
-    double upper;
-    int st = find_upper_limit(max_pend, base_ll, &upper);
-    if (st) return st;
+    // base_ll (brent kind -1), then find_upper_limit, three_tax.ml:121-163, by
+    // Brent (kind 2).  The prior is never 0 at the ML pendant length for an
+    // exponential prior short of exp underflow, handled as the reference does.
+    double base_ll = 0., upper = 0.;
+#pragma unroll 1
+    for (int kind = -1;; kind = 2) {
+      const double pend = pend_bl;
+      if (kind == 2) {
+        base_ll = last_ll;
+        if (wave_true(prior(pend) == 0.)) {
+          upper = pend;
+#pragma unroll 1
+          for (double next = upper / 2.; !wave_true(prior(next) > exp(-10.)); next = upper / 2.) upper = next;
+          break;
+        }
+        up_target = scalar(-10. + base_ll + log(prior(pend)));
+      }
+      const double start = kind < 0 ? pend : pend + (max_pend - pend) / 2.;
+      const int st = brent(kind, start, pend, max_pend, 0.02, 10, &upper);
+      if (st == ST_GSL) upper = max_pend;  // Gsl_exn EINVAL
+      else if (st) return st;
+      if (kind == 2) break;
+    }
+    upper = scalar(upper);
+    const double cut_bl = scalar(dist_bl + prox_bl);
     LaneStore s_in, s_out;
 #pragma unroll 1
     for (int n_exceptions = 0;; n_exceptions++) {
@@ -392,27 +439,19 @@ struct ThreeTaxControl {
         if (q != QNG_OK) { err = 1; fail = q; }
         return r;
       };
-      double v;
-      if (fabs(cut_bl - 0.) < 1e-5) {  // cut_bl =~ 0. (ppatteries.ml:96)
-        const double prox = (dist_bl + prox_bl) - cut_bl / 2.;
-        if (!(prox >= 0.)) return ST_ASSERT;
-        dist_bl = cut_bl / 2.;
+      auto outer = [&](double dist, int &err) -> double {
+        const double prox = (dist_bl + prox_bl) - dist;
+        if (wave_true(!(prox >= 0.))) { err = 1; fail = QNG_ASSERT; return 0.; }
+        dist_bl = dist;
         prox_bl = prox;
-        int err = 0;
-        v = inner_integral(err);
-      } else {
-        auto outer = [&](double dist, int &err) -> double {
-          const double prox = (dist_bl + prox_bl) - dist;
-          if (!(prox >= 0.)) { err = 1; fail = QNG_ASSERT; return 0.; }
-          dist_bl = dist;
-          prox_bl = prox;
-          return inner_integral(err);
-        };
-        double r;
-        const int q = qng(outer, 0., cut_bl, rel_err, s_out, &r);
-        if (q != QNG_OK && q != QNG_ABORT) fail = q;
-        v = r / cut_bl;
-      }
+        return inner_integral(err);
+      };
+      // cut_bl =~ 0. (ppatteries.ml:96): the inner integral at the edge's middle
+      const bool no_edge = wave_true(fabs(cut_bl - 0.) < 1e-5);
+      double v;
+      const int q = qng(outer, 0., cut_bl, rel_err, s_out, &v, no_edge);
+      if (q != QNG_OK && q != QNG_ABORT) fail = q;
+      if (!no_edge) v = v / cut_bl;
       if (fail == QNG_OK) { *marg = base_ll + log(v); return ST_OK; }
       if (fail == QNG_ASSERT) return ST_ASSERT;
       if (fail != QNG_ETOL) return ST_GSL;  // an uncaught Gsl_exn (EBADTOL)

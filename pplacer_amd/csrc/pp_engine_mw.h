@@ -32,9 +32,9 @@
 // (exp(rate*bl*l_k)*x[i][k])*xit[j][k].  The FP64 form rounds every product
 // and sum separately (-ffp-contract=off) and sums the per-site logs as the
 // stub does, sequentially in masked-site order (linear_c.c:416-419): workers
-// leave each site's log in LDS and, behind one more barrier, the first worker
-// wave reproduces that sum bit for bit (wave_sequential_sum).  The FP32 form
-// uses FMAs and sums the logs (in FP64) per wave, then in wave order.
+// leave each site's log in LDS and, behind barrier B, the master wave
+// reproduces that sum bit for bit (wave_sequential_sum).  The FP32 form uses
+// FMAs and sums the logs (in FP64) per wave, then in wave order.
 #pragma once
 
 #include <climits>
@@ -61,31 +61,33 @@ struct MWShared {
   long long ipart[16];       // per-worker-wave sums of site exponents
 };
 
-// LDS of one workgroup: shared header, pendant rows [n_tsl][kMaxCodes][R*4],
-// P(prox) and P(dist) [n_sl][4][4], exponential staging [3][n_sl][4], then
+// LDS of one workgroup: shared header, pendant rows [n_tsl][kMaxCodes][kT],
+// P(prox) and P(dist) [n_sl][kP], exponential staging [3][n_sl][4], then
 // per masked site (cap = the longest masked length the launch takes): the
-// site's log of a probe and the sequential sum's scratch (FP64 form), its
-// column (the masked-site list) and in the streaming form its pendant row;
-// the FP64 form also holds the sequential sum's event list.  Gamma model:
-// n_tsl = 1, n_sl = R (rate r uses slice r); Price-CAT: R = 1 and
-// n_tsl = n_sl = n_cats (a site uses its category's).
+// site's log of a probe (FP64 form, rounded up to whole blocks of 64), its
+// column (the masked-site list) and in the streaming form its pendant row.
+// Gamma model: n_tsl = 1, n_sl = R (rate r uses slice r); Price-CAT: R = 1
+// and n_tsl = n_sl = n_cats (a site uses its category's).
 template <typename Real, int R, bool STRICT>
 struct MWLayout {
   static constexpr int RS = R * 4;
   static constexpr size_t head = (sizeof(MWShared) + 15) & ~size_t(15);
+  // Reals from one pendant row, one transition-matrix slice to the next: 16
+  // bytes of padding keep the rows that a wave's lanes read at once (one per
+  // character, one per rate or category) in different banks
+  static constexpr int kPad = 16 / (int)sizeof(Real);
+  static constexpr int kT = RS + (R == 4 ? kPad : 0), kP = 16 + kPad;
   static constexpr bool strict = STRICT;  // site logs summed in site order
   int n_tsl, n_sl, cap;
   bool stream;
   __host__ __device__ MWLayout(int n_tsl_, int n_sl_, int cap_, bool stream_)
       : n_tsl(n_tsl_), n_sl(n_sl_), cap(cap_), stream(stream_) {}
-  __host__ __device__ size_t tbytes() const { return sizeof(Real) * (size_t)n_tsl * kMaxCodes * RS; }
-  __host__ __device__ size_t pbytes() const { return sizeof(Real) * (size_t)n_sl * 16; }
+  __host__ __device__ size_t tbytes() const { return sizeof(Real) * (size_t)n_tsl * kMaxCodes * kT; }
+  __host__ __device__ size_t pbytes() const { return sizeof(Real) * (size_t)n_sl * kP; }
   __host__ __device__ size_t ebytes() const { return sizeof(double) * (size_t)3 * n_sl * 4; }
   __host__ __device__ size_t off_slog() const { return head + tbytes() + 2 * pbytes() + ebytes(); }
-  __host__ __device__ size_t off_sacc() const { return off_slog() + (strict ? sizeof(double) * (size_t)cap : 0); }
-  __host__ __device__ size_t off_sev() const { return off_sacc() + (strict ? sizeof(double) * (size_t)cap : 0); }
   __host__ __device__ size_t off_sidx() const {
-    return off_sev() + (strict ? sizeof(double) * 2 * (size_t)kSeqSumEvents : 0);
+    return off_slog() + (strict ? sizeof(double) * (size_t)((cap + 63) & ~63) : 0);
   }
   __host__ __device__ size_t bytes() const { return off_sidx() + sizeof(int) * (size_t)cap * (stream ? 2 : 1); }
   __device__ Real *T(char *s) const { return reinterpret_cast<Real *>(s + head); }
@@ -95,8 +97,6 @@ struct MWLayout {
     return reinterpret_cast<double *>(s + head + tbytes() + 2 * pbytes());
   }
   __device__ double *slog(char *s) const { return reinterpret_cast<double *>(s + off_slog()); }
-  __device__ double *sacc(char *s) const { return reinterpret_cast<double *>(s + off_sacc()); }
-  __device__ double *sev(char *s) const { return reinterpret_cast<double *>(s + off_sev()); }
   __device__ int *sidx(char *s) const { return reinterpret_cast<int *>(s + off_sidx()); }
   __device__ int *sslot(char *s) const { return reinterpret_cast<int *>(s + off_sidx()) + cap; }
   static __host__ __device__ size_t align(size_t off) { return (off + 15) & ~size_t(15); }
@@ -139,9 +139,9 @@ struct MWProducts {
 // by P(prox) and P(dist) (sequential sums over j), form each (rate, state)
 // product ((pi*prox_ev)*dist_ev), hand it to keep(t, value) and accumulate
 // util = sum over (rate, state) of product*pend in that order.  pp / pd are
-// the site's P slices (for Price-CAT its category's; else rate r's slice is
-// pp + 16 r), z its evolved pendant row.
-template <typename Real, int R, bool CAT, class Keep>
+// the site's P slices (for Price-CAT, where R is 1, its category's; else rate
+// r's slice is pp + P r), z its evolved pendant row.
+template <typename Real, int R, int P, class Keep>
 __device__ __forceinline__ Real site_dist_util(const Real *pp, const Real *pd, const Real *z,
                                                const double *statd, const Real (&pO)[R * 4],
                                                const Real (&dO)[R * 4], Keep &&keep) {
@@ -151,7 +151,7 @@ __device__ __forceinline__ Real site_dist_util(const Real *pp, const Real *pd, c
   for (int r = 0; r < R; r++)
 #pragma unroll
     for (int i = 0; i < 4; i++) {
-      const Real *ppr = pp + (CAT ? 0 : r * 16) + i * 4, *pdr = pd + (CAT ? 0 : r * 16) + i * 4;
+      const Real *ppr = pp + r * P + i * 4, *pdr = pd + r * P + i * 4;
       const Real pi = (Real)statd[i];
       const int t = r * 4 + i;
       Real xv = ppr[0] * pO[r * 4], yv = pdr[0] * dO[r * 4];
@@ -169,20 +169,29 @@ __device__ __forceinline__ Real site_dist_util(const Real *pp, const Real *pd, c
   return util;
 }
 
+// Orders one wave's LDS writes before its later LDS reads of other lanes'
+// entries (LDS executes a wave's operations in order).
+__device__ __forceinline__ void wave_lds_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // CAT: Price-CAT, R == 1, site k uses P slice and pendant table sl[k] = its
 // category (site_cat); otherwise slice r for rate r and pendant table 0.
-// FP64 (strict): each active site's log goes to slog[site], and after a
-// barrier the first worker wave adds them as the stub does, in site order
-// with one rounding per term (wave_sequential_sum); FP32: the lane's logs
-// are summed and reduced per wave.
+// FP64 (strict): each site's log goes to slog (0.0 past the query's sites),
+// where the master adds them as the stub does, in site order with one
+// rounding per term (wave_sequential_sum); FP32: the lane's logs are summed
+// and reduced per wave.
 template <typename Real, int R, int SPL, bool CAT, bool STRICT>
 __device__ __forceinline__ void mw_worker(char *smem, const MWLayout<Real, R, STRICT> &lay, char *wl, int N,
                                           const uint8_t *codes, const Real *darr, const Real *parr,
                                           const int *darr_e, const int *parr_e, const int *site_cat) {
   constexpr int RS = R * 4;
   constexpr bool strict = STRICT;
-  static_assert(!CAT || R == 1, "Price-CAT GLVs have no rate axis");
+  static_assert(R == 1, "one rate; four rates take mw_worker_rates");
   static_assert(SPL >= 1, "register-resident form");
+  using L = MWLayout<Real, R, STRICT>;
   using W = MWProducts<Real, RS>;
   using Ops = RealOps<Real>;
   MWShared *sh = reinterpret_cast<MWShared *>(smem);
@@ -239,8 +248,8 @@ __device__ __forceinline__ void mw_worker(char *smem, const MWLayout<Real, R, ST
         if (op == CMD_PROBE_DIST) {
 #pragma unroll
           for (int k = 0; k < SPL; k++) {
-            const int o = CAT ? sl[k] * 16 : 0;
-            util[k] = site_dist_util<Real, R, CAT>(sPp + o, sPd + o, sT + slot[k] * RS, sh->statd, pO[k], dO[k],
+            const int o = CAT ? sl[k] * L::kP : 0;
+            util[k] = site_dist_util<Real, R, L::kP>(sPp + o, sPd + o, sT + slot[k] * L::kT, sh->statd, pO[k], dO[k],
                                                    [&](int t, Real w) { W::at(wl, wb[k], t) = w; });
           }
         } else {
@@ -248,24 +257,139 @@ __device__ __forceinline__ void mw_worker(char *smem, const MWLayout<Real, R, ST
           for (int t = 0; t < RS; t++)
 #pragma unroll
             for (int k = 0; k < SPL; k++) {
-              const Real w = W::at(wl, wb[k], t), z = sT[slot[k] * RS + t];
+              const Real w = W::at(wl, wb[k], t), z = sT[slot[k] * L::kT + t];
               util[k] = t == 0 ? w * z : Ops::madd(util[k], w, z);
             }
         }
         if constexpr (strict) {
 #pragma unroll
           for (int k = 0; k < SPL; k++)
-            if (active[k]) slog[my + k * stride] = Ops::logs(util[k]);
-          __syncthreads();  // every site's log is in slog
-          if (wv == 0) {
-            const double t = wave_sequential_sum(slog, sh->M, lay.sacc(smem), lay.sev(smem), nullptr, kSeqSumWaveMin);
-            if (lane == 0) sh->part[0] = t;
-          }
+            slog[my + k * stride] = active[k] ? Ops::logs(util[k]) : 0.0;
         } else {
           double lsum = 0.0;
 #pragma unroll
           for (int k = 0; k < SPL; k++)
             if (active[k]) lsum += Ops::logd(util[k]);
+          lsum = wave_sum(lsum);
+          if (lane == 0) sh->part[wv] = lsum;
+        }
+        __syncthreads();  // B
+        __syncthreads();  // A
+        op = sh->op;
+      }
+    }
+  }
+  // op == CMD_EXIT
+}
+
+// The worker of the four-rate gamma model.  Two layouts of a wave's 64 SPL
+// sites:
+//  * evolves (CMD_PROBE_DIST): lane 4 q + r holds rate r of sites 16 k + q, k <
+//    4 SPL.  The R quarters of a 128-byte (FP64) row sit in one quad, so a
+//    gather reads whole rows from consecutive lanes, and an entry of P is read
+//    from LDS once for 4 SPL sites instead of once per site, whose sums are
+//    independent chains.  With a lane per site the gather touched 64 lines per
+//    load and the evolve waited for LDS at each of its 16 (rate, state) pairs.
+//  * util and log: lane j owns site j (+ 64), as the sum over (rate, state) is
+//    sequential in a site.  The products pass through LDS, where they are kept
+//    for the pendant-only probes (three quarters of all) in any case.
+template <typename Real, int SPL, bool STRICT>
+__device__ __forceinline__ void mw_worker_rates(char *smem, const MWLayout<Real, 4, STRICT> &lay, char *wl, int N,
+                                                const uint8_t *codes, const Real *darr, const Real *parr,
+                                                const int *darr_e, const int *parr_e) {
+  constexpr int RS = 16, K = 4 * SPL;
+  using L = MWLayout<Real, 4, STRICT>;
+  using W = MWProducts<Real, RS>;
+  using Ops = RealOps<Real>;
+  MWShared *sh = reinterpret_cast<MWShared *>(smem);
+  const int *sidx = lay.sidx(smem);
+  double *slog = lay.slog(smem);
+  const int lane = threadIdx.x & 63;
+  const int wv = wave_id() - 1;
+  const int first = wv * 64 * SPL;  // the wave's first site
+  const int r = lane & 3, q = lane >> 2;
+  const Real *sPp = lay.Pp(smem) + r * L::kP, *sPd = lay.Pd(smem) + r * L::kP;
+  const Real *z[SPL];
+  Real pi[4];
+#pragma unroll
+  for (int i = 0; i < 4; i++) pi[i] = (Real)scalar(sh->statd[i]);
+  // products of site first + 16 k + q: this address + 16 k sites (four groups)
+  char *wq = wl + W::base(first + q) + r * 16 * (int)sizeof(Real);
+  __syncthreads();  // A
+  int op = sh->op;
+  while (op == CMD_QUERY) {
+    const int M = sh->M;
+#pragma unroll
+    for (int k = 0; k < SPL; k++) {
+      const int i = first + 64 * k + lane;
+      z[k] = lay.T(smem) + (i < M ? sh->code_slot[codes[(size_t)sh->q * N + sidx[i]]] : 0) * L::kT;
+    }
+    __syncthreads();  // B
+    __syncthreads();  // A
+    op = sh->op;
+    while (op == CMD_GATHER) {
+      const size_t row0 = (size_t)sh->loc * N;
+      Real dO[K][4], pO[K][4];
+      // sites past the query's read the row of column 0 (any valid row)
+#pragma unroll
+      for (int k = 0; k < K; k++) {
+        const int i = first + 16 * k + q;
+        const size_t at = (row0 + (i < M ? sidx[i] : 0)) * RS + r * 4;
+#pragma unroll
+        for (int j = 0; j < 4; j++) { dO[k][j] = darr[at + j]; pO[k][j] = parr[at + j]; }
+      }
+      long long es = 0;
+#pragma unroll
+      for (int k = 0; k < SPL; k++) {
+        const int i = first + 64 * k + lane;
+        if (i < M) es += (long long)darr_e[row0 + sidx[i]] + (long long)parr_e[row0 + sidx[i]];
+      }
+      es = wave_sum_ll(es);
+      if (lane == 0) sh->ipart[wv] = es;
+      __syncthreads();  // B
+      __syncthreads();  // A
+      op = sh->op;
+      while (op == CMD_PROBE || op == CMD_PROBE_DIST) {
+        if (op == CMD_PROBE_DIST) {
+#pragma unroll
+          for (int i = 0; i < 4; i++) {
+            Real pp[4], pd[4];
+#pragma unroll
+            for (int j = 0; j < 4; j++) { pp[j] = sPp[i * 4 + j]; pd[j] = sPd[i * 4 + j]; }
+#pragma unroll
+            for (int k = 0; k < K; k++) {
+              Real xv = pp[0] * pO[k][0], yv = pd[0] * dO[k][0];
+#pragma unroll
+              for (int j = 1; j < 4; j++) {
+                xv = Ops::madd(xv, pp[j], pO[k][j]);
+                yv = Ops::madd(yv, pd[j], dO[k][j]);
+              }
+              W::at(wq + k * 4 * W::kGroupBytes, 0, i) = (pi[i] * xv) * yv;
+            }
+          }
+          wave_lds_sync();  // a site's products come from its quad's lanes
+        }
+        Real util[SPL];
+#pragma unroll
+        for (int t = 0; t < RS; t++)
+#pragma unroll
+          for (int k = 0; k < SPL; k++) {
+            const Real w = W::at(wl + W::base(first + 64 * k + lane), 0, t), zt = z[k][t];
+            // the sum starts from its first product: 0 + p == p up to the sign
+            // of a zero, which no later operation can observe
+            util[k] = t == 0 ? w * zt : Ops::madd(util[k], w, zt);
+          }
+        if constexpr (STRICT) {
+#pragma unroll
+          for (int k = 0; k < SPL; k++) {
+            const int i = first + 64 * k + lane;
+            slog[i] = i < M ? Ops::logs(util[k]) : 0.0;
+          }
+        } else {
+          double lsum = 0.0;
+#pragma unroll
+          for (int k = 0; k < SPL; k++)
+            if (first + 64 * k + lane < M) lsum += Ops::logd(util[k]);
           lsum = wave_sum(lsum);
           if (lane == 0) sh->part[wv] = lsum;
         }
@@ -292,6 +416,7 @@ __device__ __forceinline__ void mw_worker_stream(char *smem, const MWLayout<Real
   constexpr int RS = R * 4;
   constexpr bool strict = STRICT;
   static_assert(!CAT || R == 1, "Price-CAT GLVs have no rate axis");
+  using L = MWLayout<Real, R, STRICT>;
   using Ops = RealOps<Real>;
   MWShared *sh = reinterpret_cast<MWShared *>(smem);
   const Real *sT = lay.T(smem), *sPp = lay.Pp(smem), *sPd = lay.Pd(smem);
@@ -306,6 +431,9 @@ __device__ __forceinline__ void mw_worker_stream(char *smem, const MWLayout<Real
   int op = sh->op;
   while (op == CMD_QUERY) {
     const int M = sh->M, q = sh->q;
+    // the sum reads whole blocks of 64: zeros past the query's sites
+    if constexpr (strict)
+      if (my < 64 && M + my < ((M + 63) & ~63)) slog[M + my] = 0.0;
     for (int i = my; i < M; i += stride) {
       const int site = sidx[i];
       const int sl = CAT ? site_cat[site] : 0;
@@ -330,7 +458,7 @@ __device__ __forceinline__ void mw_worker_stream(char *smem, const MWLayout<Real
         double lsum = 0.0;
         for (int i = my; i < M; i += stride) {
           const int slot = sslot[i];
-          const Real *z = sT + slot * RS;
+          const Real *z = sT + slot * L::kT;
           Real util;
           if (op == CMD_PROBE_DIST) {
             const int site = sidx[i];
@@ -338,8 +466,8 @@ __device__ __forceinline__ void mw_worker_stream(char *smem, const MWLayout<Real
             Real dO[RS], pO[RS];
 #pragma unroll
             for (int t = 0; t < RS; t++) { dO[t] = darr[row * RS + t]; pO[t] = parr[row * RS + t]; }
-            const int o = CAT ? (slot / kMaxCodes) * 16 : 0;
-            util = site_dist_util<Real, R, CAT>(sPp + o, sPd + o, z, sh->statd, pO, dO,
+            const int o = CAT ? (slot / kMaxCodes) * L::kP : 0;
+            util = site_dist_util<Real, R, L::kP>(sPp + o, sPd + o, z, sh->statd, pO, dO,
                                                 [&](int t, Real w) { prod[(size_t)t * cap + i] = w; });
           } else {
 #pragma unroll
@@ -351,13 +479,7 @@ __device__ __forceinline__ void mw_worker_stream(char *smem, const MWLayout<Real
           if constexpr (strict) slog[i] = Ops::logs(util);
           else lsum += Ops::logd(util);
         }
-        if constexpr (strict) {
-          __syncthreads();  // every site's log is in slog
-          if (wv == 0) {
-            const double t = wave_sequential_sum(slog, M, lay.sacc(smem), lay.sev(smem), nullptr, kSeqSumWaveMin);
-            if (lane == 0) sh->part[0] = t;
-          }
-        } else {
+        if constexpr (!strict) {
           lsum = wave_sum(lsum);
           if (lane == 0) sh->part[wv] = lsum;
         }
@@ -370,12 +492,34 @@ __device__ __forceinline__ void mw_worker_stream(char *smem, const MWLayout<Real
   // op == CMD_EXIT
 }
 
-// Orders one wave's LDS writes before its later LDS reads of other lanes'
-// entries (LDS executes a wave's operations in order).
-__device__ __forceinline__ void wave_lds_sync() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+// The informative columns of a query in order, list[0 .. cap) of them, by one
+// wave: 64 consecutive columns at a time, a column's place from the ballot of
+// those before it, eight loads in flight.  Returns how many there are (beyond
+// cap, too) and the lane's codes in `present`.
+__device__ __forceinline__ int mask_sites(const uint8_t *codes, int N, int n_inf, int cap, int *list,
+                                          unsigned &present) {
+  const int lane = threadIdx.x & 63;
+  int total = 0;
+  for (int k0 = 0; k0 < N; k0 += 512) {
+    int c[8];
+#pragma unroll
+    for (int u = 0; u < 8; u++) {
+      const int k = k0 + 64 * u + lane;
+      c[u] = k < N ? (int)codes[k] : n_inf;
+    }
+#pragma unroll
+    for (int u = 0; u < 8; u++) {
+      const bool in = c[u] < n_inf;
+      const unsigned long long m = __builtin_amdgcn_ballot_w64(in);
+      if (in) {
+        const int pos = total + (int)__builtin_popcountll(m & ~(~0ull << lane));
+        if (pos < cap) list[pos] = k0 + 64 * u + lane;
+        present |= 1u << c[u];
+      }
+      total += __builtin_popcountll(m);
+    }
+  }
+  return total;
 }
 
 // ---------------------------------------------------------------------------
@@ -402,9 +546,12 @@ struct MWMaster : ThreeTaxControl<MWMaster<Real, R, SPL, CAT, STRICT>> {
   MWShared *sh;
   Real *sT, *sPp, *sPd;
   double *sE;
+  const double *slog;
   int *sidx;
   int lane, n_workers, cap_sites, n_codes, n_inf, n_sl;
+  int n_amb;  // ambiguity codes present in the query
   double log_R;
+  double m_rate, m_l;  // the lane's rate and eigenvalue (tables)
 
   // cap: the longest masked length the launch takes (the layout's capacity)
   __device__ __forceinline__ void init(char *smem, const DevModel *dm, int cap) {
@@ -414,6 +561,7 @@ struct MWMaster : ThreeTaxControl<MWMaster<Real, R, SPL, CAT, STRICT>> {
     sPp = lay.Pp(smem);
     sPd = lay.Pd(smem);
     sE = lay.E(smem);
+    slog = lay.slog(smem);
     sidx = lay.sidx(smem);
     n_sl = dm->n_sl;
     lane = threadIdx.x & 63;
@@ -422,16 +570,16 @@ struct MWMaster : ThreeTaxControl<MWMaster<Real, R, SPL, CAT, STRICT>> {
     n_codes = dm->n_codes;
     n_inf = dm->n_inf;
     log_R = dm->log_R;
+    n_amb = 0;
+    m_rate = sh->rates[(lane >> 4) & (R - 1)];
+    m_l = sh->l[lane & 3];
     c_pend = c_dist = c_prox = __builtin_nan("");
   }
 
-  // A probe of the FP64 form has one more barrier, after which worker lane 0
-  // adds the site logs in order.
   __device__ __forceinline__ void command(int op) {
     if (lane == 0) sh->op = op;
     __syncthreads();  // A
     if (op == CMD_EXIT) return;
-    if (L::strict && (op == CMD_PROBE || op == CMD_PROBE_DIST)) __syncthreads();  // logs written
     __syncthreads();  // B
   }
 
@@ -439,29 +587,10 @@ struct MWMaster : ThreeTaxControl<MWMaster<Real, R, SPL, CAT, STRICT>> {
   // the set of characters present (their evolved rows are all a probe
   // needs), then CMD_QUERY.  Returns M.
   __device__ __forceinline__ int load_query(const uint8_t *codes, int N, int q) {
-    const int chunk = (N + 63) / 64;
-    const int lo = lane * chunk, hi = min(N, lo + chunk);
-    int cnt = 0;
     unsigned present = 0;
-    for (int k = lo; k < hi; k++) {
-      const int c = codes[k];
-      if (c < n_inf) { cnt++; present |= 1u << c; }
-    }
-    int incl = cnt;
-#pragma unroll
-    for (int m = 1; m < 64; m <<= 1) {
-      const int o = __shfl_up(incl, m, 64);
-      if (lane >= m) incl += o;
-    }
-    const int total = __builtin_amdgcn_readfirstlane(__shfl(incl, 63, 64));
+    const int total = mask_sites(codes, N, n_inf, cap_sites, sidx, present);
 #pragma unroll
     for (int m = 32; m >= 1; m >>= 1) present |= __shfl_xor(present, m, 64);
-    int pos = incl - cnt;
-    for (int k = lo; k < hi; k++)
-      if (codes[k] < n_inf) {
-        if (pos < cap_sites) sidx[pos] = k;  // a longer query is refused below
-        pos++;
-      }
     if (lane == 0) {
       int ns = 4;
       for (int c = 0; c < n_codes; c++) {
@@ -474,6 +603,7 @@ struct MWMaster : ThreeTaxControl<MWMaster<Real, R, SPL, CAT, STRICT>> {
       sh->q = q;
     }
     M = total;
+    n_amb = __builtin_popcount(__builtin_amdgcn_readfirstlane(present) >> 4);
     c_pend = __builtin_nan("");  // the pendant rows are per query
     if (total > 0 && total <= cap_sites) command(CMD_QUERY);
     return total;
@@ -489,73 +619,63 @@ struct MWMaster : ThreeTaxControl<MWMaster<Real, R, SPL, CAT, STRICT>> {
     long long es = 0;
 #pragma unroll
     for (int w = 0; w < 16; w++) es += iv[w];
-    esum = (double)es;
+    esum = scalar((double)es);
     c_dist = c_prox = __builtin_nan("");
     have_last = false;
   }
 
   // Diagd.multi_exp for the changed branch lengths and the evolved pendant
-  // rows of the characters present, with the master's 64 lanes.
+  // rows of the characters present, with the master's 64 lanes: lane r*16 +
+  // i*4 + j owns entry (i, j) of rate r's matrices.  It takes the exponential
+  // of k = j, and a quad's four exponentials reach its lanes through DPP, so
+  // nothing is staged in LDS on the probe's critical path.
+  __device__ __forceinline__ double p_entry(double e, const double (&mx)[4], const double (&mxit)[4]) const {
+    double acc = 0.0;
+    acc = acc + (dpp_f64<0x00>(e) * mx[0]) * mxit[0];
+    acc = acc + (dpp_f64<0x55>(e) * mx[1]) * mxit[1];
+    acc = acc + (dpp_f64<0xAA>(e) * mx[2]) * mxit[2];
+    acc = acc + (dpp_f64<0xFF>(e) * mx[3]) * mxit[3];
+    return acc;
+  }
   __device__ __forceinline__ void tables(bool new_pend, bool new_dist) {
     if constexpr (CAT) {
       cat_tables(new_pend, new_dist);
       return;
     }
-    // The exponentials reach the lanes forming P entries through the LDS
-    // staging area sE (one write, a wave fence, independent reads).
+    double mx[4], mxit[4];  // the lane's row of x and of xit
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+      mx[k] = sh->x[(lane & 12) + k];
+      mxit[k] = sh->xit[(lane & 3) * 4 + k];
+    }
     if (new_dist) {
-      // exp(rate_r * bl * l_k) for prox (u < 4R) and dist (4R <= u < 8R)
-      if (lane < 8 * R) {
-        const int which = lane / (4 * R), r = (lane / 4) % R, k = lane % 4;
-        sE[lane] = texp((sh->rates[r] * (which ? dist_bl : prox_bl)) * sh->l[k]);
-      }
-      wave_lds_sync();
-#pragma unroll
-      for (int base = 0; base < 2 * R * 16; base += 64) {
-        const int e = base + lane;
-        const int which = e / (R * 16), rem = e % (R * 16);
-        const int r = rem / 16, i = (rem / 4) % 4, j = rem % 4;
-        const double *ex = sE + (which * R + r) * 4;
-        double acc = 0.0;
-#pragma unroll
-        for (int k = 0; k < 4; k++) acc = acc + (ex[k] * sh->x[i * 4 + k]) * sh->xit[j * 4 + k];
-        if (e < 2 * R * 16) (which ? sPd : sPp)[rem] = (Real)acc;
+      const double p = p_entry(texp((m_rate * prox_bl) * m_l), mx, mxit);
+      const double d = p_entry(texp((m_rate * dist_bl) * m_l), mx, mxit);
+      if (lane < R * 16) {
+        sPp[(lane >> 4) * L::kP + (lane & 15)] = (Real)p;
+        sPd[(lane >> 4) * L::kP + (lane & 15)] = (Real)d;
       }
     }
     if (new_pend) {
-      double *sEp = sE + 8 * R;
-      if (lane < 4 * R) {
-        const int r = lane / 4, k = lane % 4;
-        sEp[lane] = texp((sh->rates[r] * pend_bl) * sh->l[k]);
-      }
-      wave_lds_sync();
-      // P_pend[r][i][j] at lane r*16 + i*4 + j (R*16 <= 64)
-      double pij = 0.0;
-      {
-        const int r = (lane / 16) % R, i = (lane / 4) % 4, j = lane % 4;
-        const double *ex = sEp + r * 4;
-#pragma unroll
-        for (int k = 0; k < 4; k++) pij = pij + (ex[k] * sh->x[i * 4 + k]) * sh->xit[j * 4 + k];
-      }
+      const double p = p_entry(texp((m_rate * pend_bl) * m_l), mx, mxit);
+      const int j = lane & 3, ri = (lane >> 2) & (R * 4 - 1);
       // One-hot characters: their evolved rows are columns of P (every other
       // product in gemmish_c is an exact zero), row j entry (r, i) = P[r][i][j].
-      if (lane < R * 16) {
-        const int r = lane / 16, i = (lane / 4) % 4, j = lane % 4;
-        sT[j * RS + r * 4 + i] = (Real)pij;
-      }
-      // Ambiguity codes present in the query: rows 4.. by the stub's sum.
-      const int n_t = (sh->n_slots - 4) * RS;
-      for (int base = 0; base < n_t; base += 64) {
-        const int t = base + lane;
-        const int slot = 4 + t / RS, r = (t / 4) % R, i = t % 4;
-        const int c = sh->slot_code[t < n_t ? slot : 0];
-        double acc = 0.0;
-#pragma unroll
-        for (int j = 0; j < 4; j++) {
-          const double p = __shfl(pij, r * 16 + i * 4 + j, 64);
-          acc = acc + p * sh->lv[c * 4 + j];
-        }
-        if (t < n_t) sT[slot * RS + r * 4 + i] = (Real)acc;
+      if (lane < R * 16) sT[j * L::kT + ri] = (Real)p;
+      // Ambiguity codes present in the query: rows 4.. by the stub's sum, lane
+      // j of a quad taking every fourth.
+      if (n_amb > 0) {
+        const double p0 = dpp_f64<0x00>(p), p1 = dpp_f64<0x55>(p), p2 = dpp_f64<0xAA>(p), p3 = dpp_f64<0xFF>(p);
+        if (lane < R * 16)
+          for (int slot = 4 + j; slot < 4 + n_amb; slot += 4) {
+            const double *lv = sh->lv + sh->slot_code[slot] * 4;
+            double acc = 0.0;
+            acc = acc + p0 * lv[0];
+            acc = acc + p1 * lv[1];
+            acc = acc + p2 * lv[2];
+            acc = acc + p3 * lv[3];
+            sT[slot * L::kT + ri] = (Real)acc;
+          }
       }
     }
   }
@@ -568,7 +688,7 @@ struct MWMaster : ThreeTaxControl<MWMaster<Real, R, SPL, CAT, STRICT>> {
   // summed in site order (the FP64 form), as the stubs' libm returns them;
   // the library's otherwise.
   static __device__ __forceinline__ double texp(double v) {
-    if constexpr (STRICT) return cr::exp_call(v);
+    if constexpr (STRICT) return cr::exp(v);
     else return exp(v);
   }
 
@@ -594,7 +714,7 @@ struct MWMaster : ThreeTaxControl<MWMaster<Real, R, SPL, CAT, STRICT>> {
 #pragma unroll
       for (int k = 0; k < 4; k++) acc = acc + (ex[k] * sh->x[i * 4 + k]) * sh->xit[j * 4 + k];
       if (which == 2) sT[(s * kMaxCodes + j) * 4 + i] = (Real)acc;  // one-hot row j, entry i
-      else (which ? sPd : sPp)[rem] = (Real)acc;
+      else (which ? sPd : sPp)[s * L::kP + rem % 16] = (Real)acc;
     }
     if (new_pend && sh->n_slots > 4) {
       wave_lds_sync();
@@ -612,13 +732,13 @@ struct MWMaster : ThreeTaxControl<MWMaster<Real, R, SPL, CAT, STRICT>> {
 
   // One likelihood probe (Model.log_like3 at the current three-taxon state).
   __device__ __forceinline__ double log_like() {
-    const bool new_pend = !(pend_bl == c_pend);
-    const bool new_dist = !(dist_bl == c_dist && prox_bl == c_prox);
+    const bool new_pend = wave_true(!(pend_bl == c_pend));
+    const bool new_dist = wave_true(!(dist_bl == c_dist && prox_bl == c_prox));
     tables(new_pend, new_dist);
     command(new_dist ? CMD_PROBE_DIST : CMD_PROBE);
     double tot;
     if constexpr (L::strict) {
-      tot = sh->part[0];
+      tot = wave_sequential_sum(slog, M);
     } else {
       // partials of waves >= n_workers read as 0.0; the sum is in wave order
       double pv[16];
@@ -628,14 +748,14 @@ struct MWMaster : ThreeTaxControl<MWMaster<Real, R, SPL, CAT, STRICT>> {
 #pragma unroll
       for (int w = 1; w < 16; w++) tot += pv[w];
     }
-    c_pend = pend_bl;
-    c_dist = dist_bl;
-    c_prox = prox_bl;
+    c_pend = scalar(pend_bl);
+    c_dist = scalar(dist_bl);
+    c_prox = scalar(prox_bl);
     n_calls++;
     n_probes++;
     n_dist_probes += new_dist;
     const double ll = (tot - (double)M * log_R) + PP_LOG2 * (esum + 0.0);
-    last_ll = ll;
+    last_ll = scalar(ll);
     have_last = true;
     return ll;
   }

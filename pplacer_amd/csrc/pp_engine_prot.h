@@ -255,20 +255,8 @@ struct ProtMaster : ThreeTaxControl<ProtMaster<Real, R>> {
   // mask_reindex of the query's informative sites (core.ml:25-28,146-156),
   // then CMD_QUERY.  Returns M.
   __device__ __forceinline__ int load_query(const uint8_t *codes, int N, int q) {
-    const int chunk = (N + 63) / 64;
-    const int lo = lane * chunk, hi = min(N, lo + chunk);
-    int cnt = 0;
-    for (int k = lo; k < hi; k++) cnt += codes[k] < n_inf;
-    int incl = cnt;
-#pragma unroll
-    for (int m = 1; m < 64; m <<= 1) {
-      const int o = __shfl_up(incl, m, 64);
-      if (lane >= m) incl += o;
-    }
-    const int total = __builtin_amdgcn_readfirstlane(__shfl(incl, 63, 64));
-    int pos = incl - cnt;
-    for (int k = lo; k < hi; k++)
-      if (codes[k] < n_inf) sidx[pos++] = k;
+    unsigned present = 0;
+    const int total = mask_sites(codes, N, n_inf, N, sidx, present);
     if (lane == 0) {
       sh->M = total;
       sh->q = q;
@@ -288,7 +276,7 @@ struct ProtMaster : ThreeTaxControl<ProtMaster<Real, R>> {
     long long es = 0;
 #pragma unroll
     for (int w = 0; w < 16; w++) es += iv[w];
-    esum = (double)es;
+    esum = scalar((double)es);
     c_dist = c_prox = __builtin_nan("");
     have_last = false;
   }
@@ -313,8 +301,8 @@ struct ProtMaster : ThreeTaxControl<ProtMaster<Real, R>> {
 
   // One likelihood probe (Model.log_like3 at the current three-taxon state).
   __device__ __forceinline__ double log_like() {
-    const bool new_pend = !(pend_bl == c_pend);
-    const bool new_dist = !(dist_bl == c_dist && prox_bl == c_prox);
+    const bool new_pend = wave_true(!(pend_bl == c_pend));
+    const bool new_dist = wave_true(!(dist_bl == c_dist && prox_bl == c_prox));
     tables(new_pend, new_dist);
     if (lane == 0) {
       sh->tflags = (new_dist ? 1 : 0) | (new_pend ? 2 : 0);
@@ -327,14 +315,14 @@ struct ProtMaster : ThreeTaxControl<ProtMaster<Real, R>> {
     double tot = pv[0];
 #pragma unroll
     for (int w = 1; w < 16; w++) tot += pv[w];
-    c_pend = pend_bl;
-    c_dist = dist_bl;
-    c_prox = prox_bl;
+    c_pend = scalar(pend_bl);
+    c_dist = scalar(dist_bl);
+    c_prox = scalar(prox_bl);
     n_calls++;
     n_probes++;
     n_dist_probes += new_dist;
     const double ll = (tot - (double)M * log_R) + PP_LOG2 * (esum + 0.0);
-    last_ll = ll;
+    last_ll = scalar(ll);
     have_last = true;
     return ll;
   }

@@ -4,35 +4,35 @@
 //
 // Why a wave can do it: let s_k be the sequential partial sums and u_E =
 // 2^(E-53) the spacing of doubles in the binade [2^(E-1), 2^E) (frexp
-// exponent E).  If s_{k-1} and s_k lie in the same binade E, s_{k-1} is a
-// multiple of u_E, so fl(s_{k-1} + v_k) = s_{k-1} + rint(v_k / u_E) u_E unless
-// v_k / u_E is exactly halfway between integers (then ties-to-even depends on
-// s_{k-1}).  Such a step is an exact translation by an integer number of u_E
-// that does not depend on s_{k-1}.  A run of them adds up exactly, in any
-// order, when all its steps have one sign and the run stays in the binade
-// (the integers then sum to less than 2^52).
+// exponent E).  While the partial sums stay in one binade they are multiples
+// of u_E, and adding v_k rounds to s_{k-1} + rint(v_k / u_E) u_E unless v_k /
+// u_E is exactly halfway between integers (a tie goes to even and so depends
+// on s_{k-1}).  A run of such additions moves any starting value of the
+// binade by the same multiple of u_E.
 //
-// So the wave
-//  1. splits v into 64 contiguous blocks, takes approximate prefix sums (a
-//     DPP scan of block sums) and Q = sum |v|.  Every approximate partial sum
-//     p_k is within delta = (4n + 256) 2^-53 Q of s_k (recursive summation
-//     error bounds, doubled);
-//  2. walks each block: the binade of s_k is certain when p_k is farther than
-//     delta from both binade boundaries (otherwise the wave falls back).  A
-//     step is an "event" when it is the first, changes the binade, is a tie,
-//     or moves toward zero; every other step is a translation r_k u_E, and
-//     the translations between two events are summed per block (exactly);
-//  3. numbers the events by a scan of per-lane counts, lists their term
-//     indices in event order, and adds the blocks' leading translations into
-//     the event before them (LDS atomics; exact integer multiples of one u_E,
-//     so order does not matter);
-//  4. replays the events in order on one wave-uniform value:
-//     s = (s + v_event) + translation.  The first add is the real rounding
-//     step of the sequential sum, the second is exact.
-// Sums with non-finite terms, more than kSeqSumEvents events, an uncertain
-// binade or more than 4096 terms fall back to the one-lane chain.  Each step
-// of the wave's path is a dependent FP64 operation of ~12 cycles, so below
-// kSeqSumWaveMin terms the one-lane chain is faster and is used directly.
+// So the terms are split into 64 contiguous blocks of B = ceil(n / 64), one a
+// lane, and
+//  1. a DPP scan of block sums gives each lane an approximate partial sum p
+//     before its block, within delta = (4n + 256) 2^-53 sum|v| of the true one
+//     (recursive summation error bounds, doubled);
+//  2. every lane runs the real, rounding additions of its block from p.  The
+//     block is "clean" if its terms are <= 0, none of the additions is a tie,
+//     and p and the end value, each moved delta outwards, lie in one binade:
+//     then the true partial sums lie in it too, and the block moves the true
+//     sum by exactly (end - p);
+//  3. the moves of consecutive clean blocks add up exactly (multiples of one
+//     u_E, less than 2^53 of them), in any order: a DPP scan that restarts at
+//     the other blocks;
+//  4. the other blocks (the first, those that change the binade or hold a
+//     tie; about 8 at 300 terms) are run again in order from the true sum.
+//     Whatever a block holds (mixed signs, infinities, NaN), that is the
+//     sequential sum itself, so only how many blocks are run again depends on
+//     the terms.
+//
+// What it costs: B dependent additions twice, two scans of 6 steps, and B
+// additions and two lane reads for each block run again.  On one wave: 1,700
+// cycles at 300 terms against 5,200 for the chain of one lane (17 cycles a
+// term), 1,000 against 1,900 at 100.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -41,11 +41,8 @@
 
 namespace pp {
 
-constexpr int kSeqSumEvents = 64;
-// Below this many terms the one-lane chain is the faster of the two (measured
-// on MI355X: 2,500 against 6,800 cycles at 100 terms, 8,600 against 7,400 at
-// 500, 25,000 against 19,300 at 1,600).
-constexpr int kSeqSumWaveMin = 400;
+// Longest sum the wave takes; longer ones go to the one-lane chain.
+constexpr int kSeqSumWaveMax = 4096;
 
 // 0 + v[0] + v[1] + ... + v[n-1], one lane.  A dependent chain, so it is fed
 // from LDS two blocks of eight ahead: the loads of one block are in flight
@@ -116,127 +113,124 @@ __device__ __forceinline__ double wave_scan_f64(double v) {
   return v;
 }
 
-// The binade of a partial sum s known only as p with |p - s| <= delta: its
-// frexp exponent, if s cannot lie in another binade (and is not 0).
-__device__ __forceinline__ bool certain_binade(double p, double delta, int &e) {
-  const double m = fabs(__builtin_amdgcn_frexp_mant(p));
-  e = __builtin_amdgcn_frexp_exp(p);
-  const double sc = __builtin_amdgcn_ldexp(1.0, e);
-  return ((m - 0.5) * sc > delta) & ((1.0 - m) * sc > delta) & (e > -960);
+// Inclusive prefix sums that restart at every lane set in `starts` (bit 0
+// set): lane l gets the sum from its run's first lane, the highest set bit of
+// starts up to l.  The steps of wave_scan_f64; a step's source is taken where
+// it lies in the lane's own run.
+__device__ __forceinline__ double wave_run_scan_f64(double v, unsigned long long starts) {
+  const int lane = threadIdx.x & 63;
+  const int first = 63 - __builtin_clzll(starts & (~0ull >> (63 - lane)));
+  const int back = lane - first;  // lanes of the run before this one
+  double t = dpp_f64_or0<0x111, 0xF>(v);
+  v += back >= 1 ? t : 0.0;
+  t = dpp_f64_or0<0x112, 0xF>(v);
+  v += back >= 2 ? t : 0.0;
+  t = dpp_f64_or0<0x114, 0xF>(v);
+  v += back >= 4 ? t : 0.0;
+  t = dpp_f64_or0<0x118, 0xF>(v);
+  v += back >= 8 ? t : 0.0;
+  t = dpp_f64_or0<0x142, 0xA>(v);
+  v += first < (lane & 0x30) ? t : 0.0;  // the row's run comes out of the row before
+  t = dpp_f64_or0<0x143, 0xC>(v);
+  v += first < 32 ? t : 0.0;
+  return v;
+}
+
+// The terms of a lane's block, B (wave-uniform) of them from v + lane B: in
+// registers when the block has at most CAP, else read from LDS as they are
+// needed.
+template <int CAP>
+struct SeqSumBlock {
+  const double *v;
+  int B;
+  double x[CAP > 0 ? CAP : 1];
+  __device__ __forceinline__ void load(const double *v0, int b) {
+    v = v0 + (int)(threadIdx.x & 63) * b;
+    B = b;
+#pragma unroll
+    for (int j = 0; j < CAP; j++) x[j] = v[j < B ? j : 0];
+  }
+  template <class F>
+  __device__ __forceinline__ void each(F &&f) const {
+    if constexpr (CAP > 0) {
+#pragma unroll
+      for (int j = 0; j < CAP; j++)
+        if (j < B) f(x[j]);
+    } else {
+      int j = 0;
+#pragma unroll 1
+      for (; j + 8 <= B; j += 8) {
+        double y[8];
+#pragma unroll
+        for (int i = 0; i < 8; i++) y[i] = v[j + i];
+#pragma unroll
+        for (int i = 0; i < 8; i++) f(y[i]);
+      }
+#pragma unroll 1
+      for (; j < B; j++) f(v[j]);
+    }
+  }
+};
+
+template <int CAP>
+__device__ __forceinline__ double wave_sequential_sum_of(const double *v, int n, int B, int *n_events) {
+  SeqSumBlock<CAP> blk;
+  blk.load(v, B);
+  double a = 0.0, top = -INFINITY;
+  blk.each([&](double x) {
+    a += x;
+    top = fmax(top, x);
+  });
+  const double incl = wave_scan_f64(a);
+  const double p = (threadIdx.x & 63) ? incl - a : 0.0;  // approximate partial sum before the block
+  double Q = -readlane_f64(incl, 63);
+  if (wave_true(!(top <= 0.0))) {  // not every term is <= 0
+    double q = 0.0;
+    blk.each([&](double x) { q += fabs(x); });
+    Q = wave_sum(q);
+  }
+  const double delta = (4.0 * n + 256.0) * 0x1p-53 * Q;
+  double s = p;
+  bool tie = false;
+  const double half_u = __builtin_amdgcn_ldexp(1.0, __builtin_amdgcn_frexp_exp(p) - 54);
+  blk.each([&](double x) {
+    const double t = s + x;
+    tie |= fabs(x - (t - s)) == half_u;  // the addition's exact error, in a clean block
+    s = t;
+  });
+  // (block 0 starts from p = 0: never clean)
+  const bool clean = (top <= 0.0) & !tie & (Q <= 0x1p+996) & (Q >= 0x1p-900) & (fabs(p) > delta) &
+                     (__builtin_amdgcn_frexp_exp(fabs(p) - delta) == __builtin_amdgcn_frexp_exp(fabs(s) + delta));
+  const unsigned long long again = __builtin_amdgcn_ballot_w64(!clean) | 1ull;
+  const double move = wave_run_scan_f64(clean ? s - p : 0.0, again);
+  if (n_events) *n_events = __builtin_popcountll(again);
+  double sum = readlane_f64(s, 0);  // block 0 started from 0 itself
+  const double before = dpp_f64_or0<0x138, 0xF>(move);  // of the run that ends before the lane
+#pragma unroll 1
+  for (unsigned long long rest = again & ~1ull; rest; rest &= rest - 1) {
+    double t = sum + before;  // every lane, only lane j's is the sum
+    blk.each([&](double x) { t += x; });
+    sum = readlane_f64(t, __builtin_ctzll(rest));
+  }
+  return sum + readlane_f64(move, 63);
 }
 
 // Sequential sum of v[0..n) (LDS, n wave-uniform), the same value in every
-// lane; call with the whole wave active.  acc: n doubles of LDS the wave may
-// overwrite; ev: 2 * kSeqSumEvents doubles of LDS.  v is left unchanged.
-// *n_events (when given) receives the number of events, or -1 where the sum
-// fell back to the one-lane chain.  Sums shorter than min_wave terms take the
-// one-lane chain directly.
-__device__ __forceinline__ double wave_sequential_sum(const double *v, int n, double *acc, double *ev,
-                                                      int *n_events = nullptr, int min_wave = 0) {
-  constexpr int C = 8;  // terms per LDS batch
-  const int lane = threadIdx.x & 63;
+// lane; call with the whole wave active.  v holds 64 ceil(n / 64) doubles,
+// those past n being 0.0 (adding them changes no sum).  *n_events (when
+// given) receives the number of blocks added from the true sum, or -1 where
+// the one-lane chain ran.
+__device__ __forceinline__ double wave_sequential_sum(const double *v, int n, int *n_events = nullptr) {
   if (n <= 0) {
     if (n_events) *n_events = 0;
     return 0.0;
   }
-  const int B = (n + 63) >> 6;
-  if (B <= 64 && n >= min_wave) {
-    const int lo = min(lane * B, n), hi = min(lo + B, n);
-    double a = 0.0, q = 0.0;
-    for (int c = lo; c < hi; c += C) {
-      double xs[C];
-#pragma unroll
-      for (int j = 0; j < C; j++) xs[j] = c + j < hi ? v[c + j] : 0.0;
-#pragma unroll
-      for (int j = 0; j < C; j++) {
-        a += xs[j];
-        q += fabs(xs[j]);
-      }
-    }
-    double p = wave_scan_f64(a) - a;  // approximate partial sum before the block
-    const double Q = wave_sum(q);
-    if (Q <= 0x1p+996 && Q >= 0x1p-900) {  // every term finite, not all zero
-      const double delta = (4.0 * n + 256.0) * 0x1p-53 * Q;
-      bool bad = false;
-      int prevE = 0;
-      bool prevNeg = false;
-      if (lane > 0 && lo < hi) {
-        bad = !certain_binade(p, delta, prevE);
-        prevNeg = p < 0.0;
-      }
-      unsigned long long mask = 0;  // events of the block, bit k - lo
-      double cur = 0.0, head = 0.0;
-      int curk = -1;
-      for (int c = lo; c < hi; c += C) {
-        double xs[C];
-#pragma unroll
-        for (int j = 0; j < C; j++) xs[j] = c + j < hi ? v[c + j] : 0.0;
-#pragma unroll
-        for (int j = 0; j < C; j++) {
-          const int k = c + j;
-          const bool in = k < hi;
-          const double x = xs[j];
-          p += x;
-          int E;
-          const bool cert = certain_binade(p, delta, E);
-          const double y = __builtin_amdgcn_ldexp(x, 53 - E), r = __builtin_rint(y);
-          const bool tie = fabs(y - r) == 0.5;
-          const bool toward0 = (x != 0.0) & ((x < 0.0) != prevNeg);
-          const bool ev_k = in & ((k == 0) | (E != prevE) | tie | toward0);
-          bad |= in & !cert;
-          // an event closes the translation run before it
-          const double seg = __builtin_amdgcn_ldexp(cur, prevE - 53);
-          if (ev_k & (curk >= 0)) acc[curk] = seg;
-          head = (ev_k & (curk < 0)) ? seg : head;
-          mask |= ev_k ? 1ull << (k - lo) : 0ull;
-          cur = ev_k ? 0.0 : (in ? cur + r : cur);
-          curk = ev_k ? k : curk;
-          prevE = in ? E : prevE;
-          prevNeg = in ? p < 0.0 : prevNeg;
-        }
-      }
-      if (lo < hi) {
-        const double seg = __builtin_amdgcn_ldexp(cur, prevE - 53);
-        if (curk >= 0) acc[curk] = seg;
-        else head = seg;
-      }
-      const int cnt = __popcll(mask);
-      const int incl = wave_scan_i32(cnt);
-      const int base = incl - cnt;  // this block's first event number
-      const int n_ev = __builtin_amdgcn_readlane(incl, 63);
-      if (__ballot(bad) == 0 && n_ev <= kSeqSumEvents) {
-        // pos[t] = the term index of event t
-        int *pos = reinterpret_cast<int *>(ev);
-        {
-          int j = base;
-          for (unsigned long long mm = mask; mm; mm &= mm - 1) pos[j++] = lo + __builtin_ctzll(mm);
-        }
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-        // a block's leading translation belongs to the last event before it
-        const bool has_head = (lo < hi) & (base > 0) & (head != 0.0);
-        const int kprev = has_head ? pos[base - 1] : 0;
-        const int kj = lane < n_ev ? pos[lane] : 0;
-        if (has_head) __hip_atomic_fetch_add(&acc[kprev], head, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-        const double xj = lane < n_ev ? v[kj] : 0.0;
-        const double rj = lane < n_ev ? acc[kj] : 0.0;
-        if (n_events) *n_events = n_ev;
-        double s = 0.0;
-        for (int t = 0; t < n_ev; t++) {
-          s = s + readlane_f64(xj, t);
-          s = s + readlane_f64(rj, t);
-        }
-        return s;
-      }
-    }
-  }
+  if (n <= 256) return wave_sequential_sum_of<4>(v, n, (n + 63) >> 6, n_events);
+  if (n <= 512) return wave_sequential_sum_of<8>(v, n, (n + 63) >> 6, n_events);
+  if (n <= kSeqSumWaveMax) return wave_sequential_sum_of<0>(v, n, (n + 63) >> 6, n_events);
   if (n_events) *n_events = -1;
   double s = 0.0;
-  if (lane == 0) s = ordered_sum(v, n);
+  if ((threadIdx.x & 63) == 0) s = ordered_sum(v, n);
   return readlane_f64(s, 0);
 }
 

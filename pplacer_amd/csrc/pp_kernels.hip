@@ -172,9 +172,71 @@ __device__ __forceinline__ void wave_argmin(unsigned long long &key, int &idx) {
 }
 
 // Per-edge "already pitched" flags of the baseball loop, one bit per edge:
-// lane l owns edges e = l + 64 j, bit j % 32 of word taken[(j / 32) * 64 + l]
-// (a lane reads and writes only its own words).
+// lane l owns edges e = l + 64 j, bit j % 32 of word taken[(j / 32) * 64 + l].
 __host__ __device__ __forceinline__ size_t taken_bytes(int E) { return (size_t)256 * ((E + 2047) / 2048); }
+
+// The best remaining edge of one query, on demand: the next of the stable
+// descending sort of its scores (fig.ml:143-147; a nan score sorts last but is
+// still pitched).  Lane l keeps the best untaken edge of its own, e = l + 64 j;
+// the wave's best is the minimum over lanes, and once lane w's edge is taken
+// the whole wave reads w's edges again (edge w + 64 j by lane j) for its next
+// best.  Scanning all edges at each pitch took 80,000 cycles at 3,997 edges (a
+// quarter of the FP64 baseball's time, a third of the FP32 form's).
+struct NextEdge {
+  const double *sc;
+  unsigned *taken;
+  int E, lane;
+  unsigned long long key;
+  int edge;  // INT_MAX: the lane has none left
+
+  __device__ __forceinline__ void init(const double *scores, unsigned *flags, int n_edges, int lane_) {
+    sc = scores;
+    taken = flags;
+    E = n_edges;
+    lane = lane_;
+    const int n_words = (int)(taken_bytes(E) / 256);
+    for (int w = 0; w < n_words; w++) taken[w * 64 + lane] = 0u;
+    key = ~0ull;
+    edge = INT_MAX;
+    int e = lane;
+    for (; e + 448 < E; e += 512) {  // eight scores in flight
+      double s[8];
+#pragma unroll
+      for (int u = 0; u < 8; u++) s[u] = sc[e + 64 * u];
+#pragma unroll
+      for (int u = 0; u < 8; u++) consider(desc_key(s[u]), e + 64 * u);
+    }
+    for (; e < E; e += 64) consider(desc_key(sc[e]), e);
+  }
+  __device__ __forceinline__ void consider(unsigned long long k, int e) {
+    if (k < key || (k == key && e < edge)) { key = k; edge = e; }
+  }
+  // The next edge, marked taken; INT_MAX when none is left.
+  __device__ __forceinline__ int take() {
+    unsigned long long bk = key;
+    int bi = edge;
+    wave_argmin(bk, bi);
+    bi = __builtin_amdgcn_readfirstlane(bi);
+    if (bi == INT_MAX) return bi;
+    const int w = bi & 63;
+    if (lane == w) {
+      const int j = bi >> 6;
+      taken[(j >> 5) * 64 + w] |= 1u << (j & 31);
+    }
+    wave_lds_sync();  // the flag is read by other lanes
+    bk = ~0ull;
+    int ni = INT_MAX;
+    for (int j = lane; w + 64 * j < E; j += 64) {
+      const int e = w + 64 * j;
+      if ((taken[(j >> 5) * 64 + w] >> (j & 31)) & 1u) continue;
+      const unsigned long long k = desc_key(sc[e]);
+      if (k < bk || (k == bk && e < ni)) { bk = k; ni = e; }
+    }
+    wave_argmin(bk, ni);
+    if (lane == w) { key = bk; edge = ni; }
+    return bi;
+  }
+};
 
 // Baseball over one work queue of queries, for either engine's master.
 template <class Master>
@@ -191,31 +253,14 @@ __device__ __forceinline__ void pitch_loop(const PitchArgs &a, Master &m, unsign
       if (lane == 0) { a.n_res[q] = 0; a.status[q] = M == 0 ? PP_Q_NO_INFORMATIVE : PP_Q_RANK_EXHAUSTED; }
       continue;
     }
-    const int n_words = (int)(taken_bytes(a.E) / 256);
-    for (int w = 0; w < n_words; w++) taken[w * 64 + lane] = 0u;
-    const double *sc = a.scores + (size_t)q * a.E;
+    NextEdge next;
+    next.init(a.scores + (size_t)q * a.E, taken, a.E, lane);
     double like_record = -INFINITY;
     long long n_strikes = 0, calls = 0, probes = 0, dprobes = 0;
     int n_res = 0, status = PP_Q_OK;
     for (;;) {
-      // next edge of the stable descending sort of the scores (fig.ml:143-147;
-      // a nan score sorts last but is still pitched): bi == INT_MAX is the
-      // only "none left" marker
-      unsigned long long bk = ~0ull;
-      int bi = INT_MAX;
-      for (int e = lane, j = 0; e < a.E; e += 64, j++) {
-        if ((taken[(j >> 5) * 64 + lane] >> (j & 31)) & 1u) continue;
-        const unsigned long long k = desc_key(sc[e]);
-        if (k < bk || (k == bk && e < bi)) { bk = k; bi = e; }
-      }
-      wave_argmin(bk, bi);
-      bi = __builtin_amdgcn_readfirstlane(bi);
-      if (bi == INT_MAX) break;
-      if (lane == (bi & 63)) {
-        const int j = bi >> 6;
-        taken[(j >> 5) * 64 + lane] |= 1u << (j & 31);
-      }
-      const int loc = bi;
+      const int loc = next.take();
+      if (loc == INT_MAX) break;
       m.gather(loc);
       const double cut = a.bl[loc];
       m.set_state(cut, a.start_pend, cut / 2.);
@@ -241,8 +286,8 @@ __device__ __forceinline__ void pitch_loop(const PitchArgs &a, Master &m, unsign
       const int prev_len = n_res;
       n_res++;
       if (prev_len >= a.t_max_pitches) break;
-      else if (ll > like_record) like_record = ll;
-      else if (ll < like_record - a.strike_box) {
+      else if (wave_true(ll > like_record)) like_record = scalar(ll);
+      else if (wave_true(ll < like_record - a.strike_box)) {
         if (n_strikes + 1 >= a.t_max_strikes) break;
         n_strikes++;
       }
@@ -293,6 +338,8 @@ __device__ __forceinline__ void mw_workers(char *smem, const MWLayout<Real, R, S
   if constexpr (SPL == 0) {
     Real *prod = reinterpret_cast<Real *>(scratch) + (size_t)blockIdx.x * cap * (R * 4);
     mw_worker_stream<Real, R, CAT, STRICT>(smem, lay, prod, cap, N, codes, d, p, darr_e, parr_e, site_cat);
+  } else if constexpr (R == 4) {
+    mw_worker_rates<Real, SPL, STRICT>(smem, lay, wl, N, codes, d, p, darr_e, parr_e);
   } else {
     mw_worker<Real, R, SPL, CAT, STRICT>(smem, lay, wl, N, codes, d, p, darr_e, parr_e, site_cat);
   }
