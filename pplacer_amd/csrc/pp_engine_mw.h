@@ -49,20 +49,22 @@ namespace pp {
 // CMD_PROBE_DIST: a probe whose proximal/distal lengths changed (re-evolve)
 enum { CMD_EXIT = 0, CMD_QUERY = 1, CMD_GATHER = 2, CMD_PROBE = 3, CMD_PROBE_DIST = 4 };
 
+constexpr int kNucCodes = 16;  // character codes of the 4-state models
+
 struct MWShared {
   double x[16], l[4], xit[16], statd[4], rates[kMaxRates];
-  double lv[kMaxCodes * 4];
+  double lv[kNucCodes * 4];
   int op, n_slots, M, q, loc;
   // character code -> pendant row of this query; the one-hot characters
   // (codes 0-3) always use rows 0-3
-  int code_slot[kMaxCodes];
-  int slot_code[kMaxCodes];
+  int code_slot[kNucCodes];
+  int slot_code[kNucCodes];
   double part[16];           // per-worker-wave sums of site logs
   long long ipart[16];       // per-worker-wave sums of site exponents
 };
 
-// LDS of one workgroup: shared header, pendant rows [n_tsl][kMaxCodes][kT],
-// P(prox) and P(dist) [n_sl][kP], exponential staging [3][n_sl][4], then
+// LDS of one workgroup: shared header, pendant rows [n_tsl][kTable], P(prox)
+// and P(dist) [n_sl][kP], Price-CAT's exponentials [3][n_sl][4], then
 // per masked site (cap = the longest masked length the launch takes): the
 // site's log of a probe (FP64 form, rounded up to whole blocks of 64), its
 // column (the masked-site list) and in the streaming form its pendant row.
@@ -77,14 +79,15 @@ struct MWLayout {
   // character, one per rate or category) in different banks
   static constexpr int kPad = 16 / (int)sizeof(Real);
   static constexpr int kT = RS + (R == 4 ? kPad : 0), kP = 16 + kPad;
+  static constexpr int kTable = kNucCodes * kT + (R == 4 ? 0 : 4);  // one category's pendant rows
   static constexpr bool strict = STRICT;  // site logs summed in site order
   int n_tsl, n_sl, cap;
   bool stream;
   __host__ __device__ MWLayout(int n_tsl_, int n_sl_, int cap_, bool stream_)
       : n_tsl(n_tsl_), n_sl(n_sl_), cap(cap_), stream(stream_) {}
-  __host__ __device__ size_t tbytes() const { return sizeof(Real) * (size_t)n_tsl * kMaxCodes * kT; }
+  __host__ __device__ size_t tbytes() const { return sizeof(Real) * (size_t)n_tsl * kTable; }
   __host__ __device__ size_t pbytes() const { return sizeof(Real) * (size_t)n_sl * kP; }
-  __host__ __device__ size_t ebytes() const { return sizeof(double) * (size_t)3 * n_sl * 4; }
+  __host__ __device__ size_t ebytes() const { return R == 4 ? 0 : sizeof(double) * (size_t)3 * n_sl * 4; }
   __host__ __device__ size_t off_slog() const { return head + tbytes() + 2 * pbytes() + ebytes(); }
   __host__ __device__ size_t off_sidx() const {
     return off_slog() + (strict ? sizeof(double) * (size_t)((cap + 63) & ~63) : 0);
@@ -114,7 +117,7 @@ __device__ __forceinline__ void mw_copy_model(MWShared *sh, const DevModel *dm) 
   for (int t = threadIdx.x; t < 16; t += blockDim.x) { sh->x[t] = dm->x[t]; sh->xit[t] = dm->xit[t]; }
   for (int t = threadIdx.x; t < 4; t += blockDim.x) { sh->l[t] = dm->l[t]; sh->statd[t] = dm->statd[t]; }
   for (int t = threadIdx.x; t < kMaxRates; t += blockDim.x) sh->rates[t] = dm->rates[t];
-  for (int t = threadIdx.x; t < dm->n_codes * 4; t += blockDim.x) sh->lv[t] = dm->lv[t];
+  for (int t = threadIdx.x; t < min(dm->n_codes, kNucCodes) * 4; t += blockDim.x) sh->lv[t] = dm->lv[t];
 }
 
 // ---------------------------------------------------------------------------
@@ -217,10 +220,9 @@ __device__ __forceinline__ void mw_worker(char *smem, const MWLayout<Real, R, ST
       const int i = my + k * stride;
       active[k] = i < sh->M;
       site[k] = active[k] ? sidx[i] : 0;
-      slot[k] = active[k] ? sh->code_slot[codes[(size_t)sh->q * N + site[k]]] : 0;
       sl[k] = CAT ? site_cat[site[k]] : 0;
       // pendant row of the site: table sl, character slot
-      slot[k] += sl[k] * kMaxCodes;
+      slot[k] = sl[k] * L::kTable + (active[k] ? sh->code_slot[codes[(size_t)sh->q * N + site[k]]] : 0) * L::kT;
     }
     __syncthreads();  // B
     __syncthreads();  // A
@@ -249,7 +251,7 @@ __device__ __forceinline__ void mw_worker(char *smem, const MWLayout<Real, R, ST
 #pragma unroll
           for (int k = 0; k < SPL; k++) {
             const int o = CAT ? sl[k] * L::kP : 0;
-            util[k] = site_dist_util<Real, R, L::kP>(sPp + o, sPd + o, sT + slot[k] * L::kT, sh->statd, pO[k], dO[k],
+            util[k] = site_dist_util<Real, R, L::kP>(sPp + o, sPd + o, sT + slot[k], sh->statd, pO[k], dO[k],
                                                    [&](int t, Real w) { W::at(wl, wb[k], t) = w; });
           }
         } else {
@@ -257,7 +259,7 @@ __device__ __forceinline__ void mw_worker(char *smem, const MWLayout<Real, R, ST
           for (int t = 0; t < RS; t++)
 #pragma unroll
             for (int k = 0; k < SPL; k++) {
-              const Real w = W::at(wl, wb[k], t), z = sT[slot[k] * L::kT + t];
+              const Real w = W::at(wl, wb[k], t), z = sT[slot[k] + t];
               util[k] = t == 0 ? w * z : Ops::madd(util[k], w, z);
             }
         }
@@ -437,7 +439,7 @@ __device__ __forceinline__ void mw_worker_stream(char *smem, const MWLayout<Real
     for (int i = my; i < M; i += stride) {
       const int site = sidx[i];
       const int sl = CAT ? site_cat[site] : 0;
-      sslot[i] = sh->code_slot[codes[(size_t)q * N + site]] + sl * kMaxCodes;
+      sslot[i] = sl * L::kTable + sh->code_slot[codes[(size_t)q * N + site]] * L::kT;
     }
     __syncthreads();  // B
     __syncthreads();  // A
@@ -458,7 +460,7 @@ __device__ __forceinline__ void mw_worker_stream(char *smem, const MWLayout<Real
         double lsum = 0.0;
         for (int i = my; i < M; i += stride) {
           const int slot = sslot[i];
-          const Real *z = sT + slot * L::kT;
+          const Real *z = sT + slot;
           Real util;
           if (op == CMD_PROBE_DIST) {
             const int site = sidx[i];
@@ -466,7 +468,7 @@ __device__ __forceinline__ void mw_worker_stream(char *smem, const MWLayout<Real
             Real dO[RS], pO[RS];
 #pragma unroll
             for (int t = 0; t < RS; t++) { dO[t] = darr[row * RS + t]; pO[t] = parr[row * RS + t]; }
-            const int o = CAT ? (slot / kMaxCodes) * L::kP : 0;
+            const int o = CAT ? (slot / L::kTable) * L::kP : 0;
             util = site_dist_util<Real, R, L::kP>(sPp + o, sPd + o, z, sh->statd, pO, dO,
                                                 [&](int t, Real w) { prod[(size_t)t * cap + i] = w; });
           } else {
@@ -565,7 +567,7 @@ struct MWMaster : ThreeTaxControl<MWMaster<Real, R, SPL, CAT, STRICT>> {
     sidx = lay.sidx(smem);
     n_sl = dm->n_sl;
     lane = threadIdx.x & 63;
-    n_workers = (blockDim.x >> 6) - 1;
+    n_workers = (int)(blockDim.x >> 6) - 1;
     cap_sites = cap;
     n_codes = dm->n_codes;
     n_inf = dm->n_inf;
@@ -613,12 +615,7 @@ struct MWMaster : ThreeTaxControl<MWMaster<Real, R, SPL, CAT, STRICT>> {
   __device__ __forceinline__ void gather(int loc) {
     if (lane == 0) sh->loc = loc;
     command(CMD_GATHER);
-    long long iv[16];
-#pragma unroll
-    for (int w = 0; w < 16; w++) iv[w] = w < n_workers ? sh->ipart[w] : 0;
-    long long es = 0;
-#pragma unroll
-    for (int w = 0; w < 16; w++) es += iv[w];
+    const long long es = wave_sum_ll(lane < n_workers ? sh->ipart[lane] : 0);
     esum = scalar((double)es);
     c_dist = c_prox = __builtin_nan("");
     have_last = false;
@@ -636,6 +633,22 @@ struct MWMaster : ThreeTaxControl<MWMaster<Real, R, SPL, CAT, STRICT>> {
     acc = acc + (dpp_f64<0xAA>(e) * mx[2]) * mxit[2];
     acc = acc + (dpp_f64<0xFF>(e) * mx[3]) * mxit[3];
     return acc;
+  }
+  // Ambiguity codes present in the query: entry (r, i) of rows 4.. by the
+  // stub's sum over the row's P entries p, which a quad's lanes hold; lane j
+  // takes every fourth row.  The whole wave calls; `at` is row 0's entry.
+  __device__ __forceinline__ void ambiguity_rows(double p, bool active, Real *at) const {
+    const double p0 = dpp_f64<0x00>(p), p1 = dpp_f64<0x55>(p), p2 = dpp_f64<0xAA>(p), p3 = dpp_f64<0xFF>(p);
+    if (active)
+      for (int slot = 4 + (lane & 3); slot < 4 + n_amb; slot += 4) {
+        const double *lv = sh->lv + sh->slot_code[slot] * 4;
+        double acc = 0.0;
+        acc = acc + p0 * lv[0];
+        acc = acc + p1 * lv[1];
+        acc = acc + p2 * lv[2];
+        acc = acc + p3 * lv[3];
+        at[slot * L::kT] = (Real)acc;
+      }
   }
   __device__ __forceinline__ void tables(bool new_pend, bool new_dist) {
     if constexpr (CAT) {
@@ -662,28 +675,10 @@ struct MWMaster : ThreeTaxControl<MWMaster<Real, R, SPL, CAT, STRICT>> {
       // One-hot characters: their evolved rows are columns of P (every other
       // product in gemmish_c is an exact zero), row j entry (r, i) = P[r][i][j].
       if (lane < R * 16) sT[j * L::kT + ri] = (Real)p;
-      // Ambiguity codes present in the query: rows 4.. by the stub's sum, lane
-      // j of a quad taking every fourth.
-      if (n_amb > 0) {
-        const double p0 = dpp_f64<0x00>(p), p1 = dpp_f64<0x55>(p), p2 = dpp_f64<0xAA>(p), p3 = dpp_f64<0xFF>(p);
-        if (lane < R * 16)
-          for (int slot = 4 + j; slot < 4 + n_amb; slot += 4) {
-            const double *lv = sh->lv + sh->slot_code[slot] * 4;
-            double acc = 0.0;
-            acc = acc + p0 * lv[0];
-            acc = acc + p1 * lv[1];
-            acc = acc + p2 * lv[2];
-            acc = acc + p3 * lv[3];
-            sT[slot * L::kT + ri] = (Real)acc;
-          }
-      }
+      if (n_amb > 0) ambiguity_rows(p, lane < R * 16, sT + ri);
     }
   }
 
-  // Price-CAT tables: the same sums for every category slice, staged through
-  // LDS (more entries than lanes): exponentials, then P(prox), P(dist) and
-  // P(pend) entries; the one-hot pendant rows are P(pend) columns and the
-  // ambiguity rows are formed from them.
   // The exponentials of P(t): correctly rounded where the site logs are
   // summed in site order (the FP64 form), as the stubs' libm returns them;
   // the library's otherwise.
@@ -692,40 +687,49 @@ struct MWMaster : ThreeTaxControl<MWMaster<Real, R, SPL, CAT, STRICT>> {
     else return exp(v);
   }
 
+  // Price-CAT tables: the same sums for every category slice.  The
+  // exponentials (category s, eigenvalue k at 4 s + k) go through LDS, a lane
+  // one of 64 at a time, so each is taken once; then lane (s mod 4) 16 + i 4 +
+  // j forms entry (i, j) of every fourth category's matrices, with its rows of
+  // x and xit in registers, and the ambiguity rows from its quad.
+  __device__ __forceinline__ void cat_exps(double bl, double *e) {
+    for (int t = lane; t < 4 * n_sl; t += 64) e[t] = texp((sh->rates[t >> 2] * bl) * m_l);
+  }
+  static __device__ __forceinline__ double cat_entry(const double *e, const double (&mx)[4], const double (&mxit)[4]) {
+    double acc = 0.0;
+#pragma unroll
+    for (int k = 0; k < 4; k++) acc = acc + (e[k] * mx[k]) * mxit[k];
+    return acc;
+  }
   __device__ __forceinline__ void cat_tables(bool new_pend, bool new_dist) {
-    const int nd = new_dist ? 2 * n_sl * 4 : 0, np = new_pend ? n_sl * 4 : 0;
-    // sE[0 .. 2 n_sl 4): prox then dist; sE[2 n_sl 4 ..): pend
-    for (int t = lane; t < nd + np; t += 64) {
-      const bool pend = t >= nd;
-      const int u = pend ? t - nd : t;
-      const int which = pend ? 2 : u / (n_sl * 4), rem = u % (n_sl * 4), s = rem / 4, k = rem % 4;
-      const double bl = which == 0 ? prox_bl : which == 1 ? dist_bl : pend_bl;
-      sE[which * n_sl * 4 + rem] = texp((sh->rates[s] * bl) * sh->l[k]);
+    double *e0 = sE, *e1 = sE + 4 * n_sl, *e2 = sE + 8 * n_sl;  // proximal, distal, pendant
+    if (new_dist) {
+      cat_exps(prox_bl, e0);
+      cat_exps(dist_bl, e1);
     }
+    if (new_pend) cat_exps(pend_bl, e2);
     wave_lds_sync();
-    const int ndp = new_dist ? 2 * n_sl * 16 : 0, npp = new_pend ? n_sl * 16 : 0;
-    for (int t = lane; t < ndp + npp; t += 64) {
-      const bool pend = t >= ndp;
-      const int u = pend ? t - ndp : t;
-      const int which = pend ? 2 : u / (n_sl * 16), rem = u % (n_sl * 16);
-      const int s = rem / 16, i = (rem / 4) % 4, j = rem % 4;
-      const double *ex = sE + (which * n_sl + s) * 4;
-      double acc = 0.0;
+    double mx[4], mxit[4];
 #pragma unroll
-      for (int k = 0; k < 4; k++) acc = acc + (ex[k] * sh->x[i * 4 + k]) * sh->xit[j * 4 + k];
-      if (which == 2) sT[(s * kMaxCodes + j) * 4 + i] = (Real)acc;  // one-hot row j, entry i
-      else (which ? sPd : sPp)[s * L::kP + rem % 16] = (Real)acc;
+    for (int k = 0; k < 4; k++) {
+      mx[k] = sh->x[(lane & 12) + k];
+      mxit[k] = sh->xit[(lane & 3) * 4 + k];
     }
-    if (new_pend && sh->n_slots > 4) {
-      wave_lds_sync();
-      const int n_amb = sh->n_slots - 4;
-      for (int t = lane; t < n_sl * n_amb * 4; t += 64) {
-        const int s = t / (n_amb * 4), slot = 4 + (t / 4) % n_amb, i = t % 4;
-        const int c = sh->slot_code[slot];
-        double acc = 0.0;
-#pragma unroll
-        for (int j = 0; j < 4; j++) acc = acc + (double)sT[(s * kMaxCodes + j) * 4 + i] * sh->lv[c * 4 + j];
-        sT[(s * kMaxCodes + slot) * 4 + i] = (Real)acc;
+    const int i = (lane >> 2) & 3, j = lane & 3;
+    if (new_dist) {
+#pragma unroll 2
+      for (int s = lane >> 4; s < n_sl; s += 4) {
+        sPp[s * L::kP + (lane & 15)] = (Real)cat_entry(e0 + 4 * s, mx, mxit);
+        sPd[s * L::kP + (lane & 15)] = (Real)cat_entry(e1 + 4 * s, mx, mxit);
+      }
+    }
+    if (new_pend) {
+#pragma unroll 2
+      for (int s0 = 0; s0 < n_sl; s0 += 4) {  // whole waves: quads exchange entries
+        const int s = s0 + (lane >> 4);
+        const double p = cat_entry(e2 + 4 * (s < n_sl ? s : 0), mx, mxit);
+        if (s < n_sl) sT[s * L::kTable + j * 4 + i] = (Real)p;  // one-hot row j, entry i
+        if (n_amb > 0) ambiguity_rows((double)(Real)p, s < n_sl, sT + s * L::kTable + i);
       }
     }
   }
@@ -740,13 +744,9 @@ struct MWMaster : ThreeTaxControl<MWMaster<Real, R, SPL, CAT, STRICT>> {
     if constexpr (L::strict) {
       tot = wave_sequential_sum(slog, M);
     } else {
-      // partials of waves >= n_workers read as 0.0; the sum is in wave order
-      double pv[16];
-#pragma unroll
-      for (int w = 0; w < 16; w++) pv[w] = w < n_workers ? sh->part[w] : 0.0;
-      tot = pv[0];
-#pragma unroll
-      for (int w = 1; w < 16; w++) tot += pv[w];
+      const double pv = sh->part[lane & 15];  // lane w: worker wave w's partial, added in wave order
+      tot = readlane_f64(pv, 0);
+      for (int w = 1; w < n_workers; w++) tot += readlane_f64(pv, w);
     }
     c_pend = scalar(pend_bl);
     c_dist = scalar(dist_bl);

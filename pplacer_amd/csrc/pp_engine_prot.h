@@ -270,12 +270,7 @@ struct ProtMaster : ThreeTaxControl<ProtMaster<Real, R>> {
   __device__ __forceinline__ void gather(int loc) {
     if (lane == 0) sh->loc = loc;
     command(CMD_GATHER);
-    long long iv[16];
-#pragma unroll
-    for (int w = 0; w < 16; w++) iv[w] = w < n_workers ? sh->ipart[w] : 0;
-    long long es = 0;
-#pragma unroll
-    for (int w = 0; w < 16; w++) es += iv[w];
+    const long long es = wave_sum_ll(lane < n_workers ? sh->ipart[lane] : 0);
     esum = scalar((double)es);
     c_dist = c_prox = __builtin_nan("");
     have_last = false;
@@ -309,12 +304,9 @@ struct ProtMaster : ThreeTaxControl<ProtMaster<Real, R>> {
       sh->tile_next = 0;
     }
     command(new_dist ? CMD_PROBE_DIST : CMD_PROBE);
-    double pv[16];
-#pragma unroll
-    for (int w = 0; w < 16; w++) pv[w] = w < n_workers ? sh->part[w] : 0.0;
-    double tot = pv[0];
-#pragma unroll
-    for (int w = 1; w < 16; w++) tot += pv[w];
+    const double pv = sh->part[lane & 15];  // lane w: worker wave w's partial, added in wave order
+    double tot = readlane_f64(pv, 0);
+    for (int w = 1; w < n_workers; w++) tot += readlane_f64(pv, w);
     c_pend = scalar(pend_bl);
     c_dist = scalar(dist_bl);
     c_prox = scalar(prox_bl);

@@ -351,8 +351,7 @@ void pitch_mw_kernel(PitchArgs a) {
   extern __shared__ __align__(16) char smem[];
   const int cap = mw_cap<SPL>(a.cap_sites);
   const MWLayout<Real, R, STRICT> lay = mw_layout<Real, R, STRICT>(a.model, cap, SPL == 0);
-  MWShared *sh = reinterpret_cast<MWShared *>(smem);
-  mw_copy_model(sh, a.model);
+  mw_copy_model(reinterpret_cast<MWShared *>(smem), a.model);
   __syncthreads();
   unsigned *taken = reinterpret_cast<unsigned *>(smem + lay.align(lay.bytes()));
   if (wave_id() != 0) {
@@ -558,8 +557,7 @@ void optimize_mw_kernel(OptArgs a) {
   extern __shared__ __align__(16) char smem[];
   const int cap = mw_cap<SPL>(a.cap_sites);
   const MWLayout<Real, R, STRICT> lay = mw_layout<Real, R, STRICT>(a.model, cap, SPL == 0);
-  MWShared *sh = reinterpret_cast<MWShared *>(smem);
-  mw_copy_model(sh, a.model);
+  mw_copy_model(reinterpret_cast<MWShared *>(smem), a.model);
   __syncthreads();
   if (wave_id() != 0) {
     char *wl = smem + lay.align(lay.bytes());
