@@ -809,6 +809,18 @@ size_t prot_scratch_bytes(int cap_pairs) {
   return sizeof(double) * ProtLayout::scratch_reals(cap_pairs);
 }
 
+// Room in the FP64 engine's LDS (one workgroup a CU) for one round's G behind
+// `lds` bytes of layout and flags: sets *lds_g to its offset and returns the
+// launch's LDS.  FP32: none.
+template <typename Real>
+size_t prot_lds_with_g(const pp_ctx *c, size_t lds, int *lds_g) {
+  const size_t at = ProtLayout::align(lds), end = at + prot_round_bytes(kProtBlock - 64);
+  *lds_g = 0;
+  if (std::is_same<Real, float>::value || end > c->max_lds) return lds;
+  *lds_g = (int)at;
+  return end;
+}
+
 // Scratch of a 20-state kernel's full-occupancy grid.
 template <typename Real, int R>
 size_t prot_scratch_need(const pp_ctx *c, const void *kern, size_t lds) {
@@ -854,7 +866,7 @@ int prot_scratch(pp_ctx *c, const void *kern, size_t lds, int cap_pairs, void **
 
 template <typename Real, int R>
 int launch_pitch_prot(pp_ctx *c, PitchArgs a) {
-  const size_t lds = prot_lds<Real, R>(c) + taken_bytes(c->E);
+  const size_t lds = prot_lds_with_g<Real>(c, prot_lds<Real, R>(c) + taken_bytes(c->E), &a.lds_g);
   const void *k = reinterpret_cast<const void *>(&pitch_prot_kernel<Real, R>);
   const int grid = occupancy_grid<Real, R>(k, kProtBlock, lds, c->n_cu, a.nq);
   a.cap_pairs = prot_cap_pairs<Real, R>(c);
@@ -867,7 +879,7 @@ int launch_pitch_prot(pp_ctx *c, PitchArgs a) {
 
 template <typename Real, int R>
 int launch_opt_prot(pp_ctx *c, OptArgs a) {
-  const size_t lds = prot_lds<Real, R>(c);
+  const size_t lds = prot_lds_with_g<Real>(c, prot_lds<Real, R>(c), &a.lds_g);
   const void *k = reinterpret_cast<const void *>(&optimize_prot_kernel<Real, R>);
   const int grid = occupancy_grid<Real, R>(k, kProtBlock, lds, c->n_cu, a.n_jobs);
   a.cap_pairs = prot_cap_pairs<Real, R>(c);
@@ -880,7 +892,7 @@ int launch_opt_prot(pp_ctx *c, OptArgs a) {
 
 template <int R>
 int launch_marg_prot(pp_ctx *c, OptArgs a) {
-  const size_t lds = prot_lds<double, R>(c);
+  const size_t lds = prot_lds_with_g<double>(c, prot_lds<double, R>(c), &a.lds_g);
   const void *k = reinterpret_cast<const void *>(&marginal_prot_kernel<R>);
   const int grid = occupancy_grid<double, R>(k, kProtBlock, lds, c->n_cu, a.n_jobs);
   a.cap_pairs = prot_cap_pairs<double, R>(c);

@@ -63,6 +63,7 @@ struct PitchArgs {
   // 4-state streaming form: per-workgroup products [R*4][cap_sites]
   void *scratch;
   int cap_pairs, cap_sites;
+  int lds_g;            // FP64 20-state engine: LDS offset of one round's G (0: none)
   const int *site_cat;  // Price-CAT: category of each pre-masked site (else nullptr)
 };
 
@@ -99,6 +100,7 @@ struct OptArgs {
   unsigned long long *n_calls;  // [0]: likelihood calls; [2], [3]: as in PitchArgs
   void *scratch;                // as in PitchArgs
   int cap_pairs, cap_sites;
+  int lds_g;                    // as in PitchArgs
   const int *site_cat;          // as in PitchArgs
   // marginal likelihoods (-p): mode 1 writes kept[].marg, mode 0 out_ll
   double pp_rel_err;

@@ -383,6 +383,7 @@ __device__ __forceinline__ size_t prot_setup(char *smem, const DevModel *dm, int
 
 template <typename Real, int R, class Args>
 __device__ __forceinline__ void prot_workers(char *smem, const Args &a) {
+  double *lds_g = a.lds_g ? reinterpret_cast<double *>(smem + a.lds_g) : nullptr;
   if constexpr (std::is_same<Real, float>::value) {
     float *scr = reinterpret_cast<float *>(a.scratch) +
                  Prot32Layout<R>::scratch_floats(a.cap_pairs / 64) * blockIdx.x;
@@ -390,8 +391,9 @@ __device__ __forceinline__ void prot_workers(char *smem, const Args &a) {
                      reinterpret_cast<const float *>(a.parr), a.darr_e, a.parr_e);
   } else {
     double *scr = reinterpret_cast<double *>(a.scratch) + ProtLayout::scratch_reals(a.cap_pairs) * blockIdx.x;
-    prot_worker<double, R>(smem, scr, a.cap_pairs, a.N, a.codes, reinterpret_cast<const double *>(a.darr),
-                           reinterpret_cast<const double *>(a.parr), a.darr_e, a.parr_e, a.site_cat);
+    prot_worker<R>(smem, scr, a.cap_pairs, a.N, a.codes, reinterpret_cast<const double *>(a.darr),
+                   reinterpret_cast<const double *>(a.parr), a.darr_e, a.parr_e, a.site_cat, a.model,
+                   lds_g);
   }
 }
 
@@ -609,9 +611,7 @@ __global__ __launch_bounds__(512) void marginal_prot_kernel(OptArgs a) {
   prot_copy_model(reinterpret_cast<ProtShared *>(smem), a.model);
   __syncthreads();
   if (wave_id() != 0) {
-    double *scr = reinterpret_cast<double *>(a.scratch) + ProtLayout::scratch_reals(a.cap_pairs) * blockIdx.x;
-    prot_worker<double, R>(smem, scr, a.cap_pairs, a.N, a.codes, reinterpret_cast<const double *>(a.darr),
-                           reinterpret_cast<const double *>(a.parr), a.darr_e, a.parr_e, a.site_cat);
+    prot_workers<double, R>(smem, a);
     return;
   }
   ProtMaster<double, R> m;
