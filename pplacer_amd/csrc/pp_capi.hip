@@ -258,11 +258,12 @@ int make_fp32_copies(pp_ctx *c) {
   ENSURE(c->b_p32, (size_t)G * N * RS, &p32);
   ENSURE(c->b_de32, (size_t)G * N, &de32);
   ENSURE(c->b_pe32, (size_t)G * N, &pe32);
+  const int G4 = RS / 4;  // R or 5 R, R at most 32
   const dim3 grid(4096), block(256);
   hipLaunchKernelGGL(fp32_rescale_kernel, grid, block, 0, c->stream, (const double *)c->b_d64.p,
-                     (const int *)c->b_de.p, d32, de32, (long)G * N, RS);
+                     (const int *)c->b_de.p, d32, de32, (long)G * N, G4);
   hipLaunchKernelGGL(fp32_rescale_kernel, grid, block, 0, c->stream, (const double *)c->b_p64.p,
-                     (const int *)c->b_pe.p, p32, pe32, (long)G * N, RS);
+                     (const int *)c->b_pe.p, p32, pe32, (long)G * N, G4);
   HIPCHECK(hipGetLastError());
   HIPCHECK(hipStreamSynchronize(c->stream));
   return PP_OK;
@@ -2203,10 +2204,7 @@ static int twin_logdot(const double *statd, const double *x, const double *y, co
   uint16_t *dm = mask ? s.up(mask, N) : nullptr;
   double *du = s.up<double>(nullptr, std::max(n_used, 1)), *dout = s.up<double>(nullptr, 1);
   CHECK(dx && dy && du && dout, PP_ENOMEM, "device allocation failed");
-  if (n_used > 0)
-    hipLaunchKernelGGL(util_kernel, dim3((n_used + 255) / 256), dim3(256), 0, 0, du, ds, dx, dy, dz, dm, first,
-                       n_used, R, N, S);
-  hipLaunchKernelGGL(logsum_kernel, dim3(1), dim3(64), 0, 0, du, dm, first, n_used, R, rate_term, dout);
+  launch_logsum(0, du, ds, dx, dy, dz, dm, first, n_used, R, N, S, rate_term, nullptr, nullptr, nullptr, dout);
   HIPCHECK(hipGetLastError());
   HIPCHECK(hipMemcpy(out, dout, 8, hipMemcpyDeviceToHost));
   if (util && n_used > 0) HIPCHECK(hipMemcpy(util, du, (size_t)n_used * 8, hipMemcpyDeviceToHost));
