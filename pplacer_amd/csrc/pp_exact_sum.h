@@ -44,11 +44,10 @@ namespace pp {
 // Longest sum the wave takes; longer ones go to the one-lane chain.
 constexpr int kSeqSumWaveMax = 4096;
 
-// 0 + v[0] + v[1] + ... + v[n-1], one lane.  A dependent chain, so it is fed
+// s + v[0] + v[1] + ... + v[n-1], one lane.  A dependent chain, so it is fed
 // from LDS two blocks of eight ahead: the loads of one block are in flight
 // while the previous block is added.
-__device__ __forceinline__ double ordered_sum(const double *v, int n) {
-  double s = 0.0;
+__device__ __forceinline__ double ordered_sum(const double *v, int n, double s = 0.0) {
   double a[8], b[8];
 #pragma unroll
   for (int j = 0; j < 8; j++) a[j] = j < n ? v[j] : 0.0;
@@ -173,7 +172,7 @@ struct SeqSumBlock {
 };
 
 template <int CAP>
-__device__ __forceinline__ double wave_sequential_sum_of(const double *v, int n, int B, int *n_events) {
+__device__ __forceinline__ double wave_sequential_sum_of(const double *v, int n, int B, int *n_events, double start) {
   SeqSumBlock<CAP> blk;
   blk.load(v, B);
   double a = 0.0, top = -INFINITY;
@@ -182,12 +181,12 @@ __device__ __forceinline__ double wave_sequential_sum_of(const double *v, int n,
     top = fmax(top, x);
   });
   const double incl = wave_scan_f64(a);
-  const double p = (threadIdx.x & 63) ? incl - a : 0.0;  // approximate partial sum before the block
-  double Q = -readlane_f64(incl, 63);
+  const double p = (threadIdx.x & 63) ? start + (incl - a) : start;  // approximate partial sum before the block
+  double Q = -(start + readlane_f64(incl, 63));
   if (wave_true(!(top <= 0.0))) {  // not every term is <= 0
     double q = 0.0;
     blk.each([&](double x) { q += fabs(x); });
-    Q = wave_sum(q);
+    Q = wave_sum(q) + fabs(start);
   }
   const double delta = (4.0 * n + 256.0) * 0x1p-53 * Q;
   double s = p;
@@ -198,13 +197,12 @@ __device__ __forceinline__ double wave_sequential_sum_of(const double *v, int n,
     tie |= fabs(x - (t - s)) == half_u;  // the addition's exact error, in a clean block
     s = t;
   });
-  // (block 0 starts from p = 0: never clean)
-  const bool clean = (top <= 0.0) & !tie & (Q <= 0x1p+996) & (Q >= 0x1p-900) & (fabs(p) > delta) &
+  const bool clean = ((threadIdx.x & 63) != 0) & (top <= 0.0) & (start <= 0.0) & !tie & (Q <= 0x1p+996) & (Q >= 0x1p-900) & (fabs(p) > delta) &
                      (__builtin_amdgcn_frexp_exp(fabs(p) - delta) == __builtin_amdgcn_frexp_exp(fabs(s) + delta));
   const unsigned long long again = __builtin_amdgcn_ballot_w64(!clean) | 1ull;
   const double move = wave_run_scan_f64(clean ? s - p : 0.0, again);
   if (n_events) *n_events = __builtin_popcountll(again);
-  double sum = readlane_f64(s, 0);  // block 0 started from 0 itself
+  double sum = readlane_f64(s, 0);  // block 0 started from the true sum itself
   const double before = dpp_f64_or0<0x138, 0xF>(move);  // of the run that ends before the lane
 #pragma unroll 1
   for (unsigned long long rest = again & ~1ull; rest; rest &= rest - 1) {
@@ -217,20 +215,22 @@ __device__ __forceinline__ double wave_sequential_sum_of(const double *v, int n,
 
 // Sequential sum of v[0..n) (LDS, n wave-uniform), the same value in every
 // lane; call with the whole wave active.  v holds 64 ceil(n / 64) doubles,
-// those past n being 0.0 (adding them changes no sum).  *n_events (when
-// given) receives the number of blocks added from the true sum, or -1 where
-// the one-lane chain ran.
-__device__ __forceinline__ double wave_sequential_sum(const double *v, int n, int *n_events = nullptr) {
+// those past n being 0.0 (adding them changes no sum).  The sum goes on from
+// `start` (a longer sum in pieces; not -0.0).  *n_events (when given) receives
+// the number of blocks added from the true sum, or -1 where the one-lane chain
+// ran.
+__device__ __forceinline__ double wave_sequential_sum(const double *v, int n, int *n_events = nullptr,
+                                                      double start = 0.0) {
   if (n <= 0) {
     if (n_events) *n_events = 0;
-    return 0.0;
+    return start;
   }
-  if (n <= 256) return wave_sequential_sum_of<4>(v, n, (n + 63) >> 6, n_events);
-  if (n <= 512) return wave_sequential_sum_of<8>(v, n, (n + 63) >> 6, n_events);
-  if (n <= kSeqSumWaveMax) return wave_sequential_sum_of<0>(v, n, (n + 63) >> 6, n_events);
+  if (n <= 256) return wave_sequential_sum_of<4>(v, n, (n + 63) >> 6, n_events, start);
+  if (n <= 512) return wave_sequential_sum_of<8>(v, n, (n + 63) >> 6, n_events, start);
+  if (n <= kSeqSumWaveMax) return wave_sequential_sum_of<0>(v, n, (n + 63) >> 6, n_events, start);
   if (n_events) *n_events = -1;
   double s = 0.0;
-  if ((threadIdx.x & 63) == 0) s = ordered_sum(v, n);
+  if ((threadIdx.x & 63) == 0) s = ordered_sum(v, n, start);
   return readlane_f64(s, 0);
 }
 

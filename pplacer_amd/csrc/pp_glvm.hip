@@ -110,23 +110,6 @@ __global__ void evolve_kernel(double *dst, const double *src, const double *P, i
   }
 }
 
-// Sums of the exponents as the OCaml accumulates them, one float addition per
-// site in site order (total_twoexp / masked_total_twoexp /
-// bounded_total_twoexp, gstar_support.ml:47-70), combined with the tensor
-// part: out = t + log 2 * ((sum x + sum y) + sum z) (z optional).
-__global__ void finish_logdot_kernel(const double *t, const int *xe, const int *ye, const int *ze,
-                                     const uint16_t *mask, int first, int last, double *out) {
-  if (threadIdx.x != 0 || blockIdx.x != 0) return;
-  double tx = 0., ty = 0., tz = 0.;
-  for (int i = first; i <= last; i++) {
-    if (mask && !mask[i]) continue;
-    tx = tx + (double)xe[i];
-    ty = ty + (double)ye[i];
-    if (ze) tz = tz + (double)ze[i];
-  }
-  *out = *t + PP_LOG2 * (ze ? (tx + ty) + tz : tx + ty);
-}
-
 // site_log_like_arr3 (gmix_model.ml:323-345); a site whose likelihood is not
 // positive is reported in *bad (the smallest such site)
 __global__ void site_log_like_kernel(const double *statd, const double *x, const double *y, const double *z,
@@ -205,14 +188,11 @@ int logdot_impl(const pp_glv *x, const pp_glv *y, const uint16_t *mask, int firs
   const int n_used = last - first + 1;
   Scratch s;
   uint16_t *dm = mask ? s.up(mask, (size_t)x->N) : nullptr;
-  double *du = s.up<double>(nullptr, n_used), *dt = s.up<double>(nullptr, 2);
+  double *du = s.up<double>(nullptr, n_used), *dt = s.up<double>(nullptr, 1);
   CHECK(du && dt && (dm || !mask), PP_ENOMEM, "device allocation failed");
-  hipLaunchKernelGGL(util_kernel, dim3((n_used + 255) / 256), dim3(256), 0, c->stream, du, nullptr, x->a, y->a,
-                     nullptr, dm, first, n_used, x->R, x->N, x->S);
-  hipLaunchKernelGGL(logsum_kernel, dim3(1), dim3(64), 0, c->stream, du, dm, first, n_used, x->R, 1, dt);
-  hipLaunchKernelGGL(gv::finish_logdot_kernel, dim3(1), dim3(1), 0, c->stream, dt, x->e, y->e, nullptr, dm, first,
-                     last, dt + 1);
-  return fetch_double(c, dt + 1, out);
+  launch_logsum(c->stream, du, nullptr, x->a, y->a, nullptr, dm, first, n_used, x->R, x->N, x->S, 1, x->e, y->e, nullptr,
+                dt);
+  return fetch_double(c, dt, out);
 }
 
 }  // namespace gv
@@ -449,14 +429,10 @@ int pp_gmix_log_like3(pp_ctx *ctx, const pp_glv *x, const pp_glv *y, const pp_gl
   HIPCHECK(hipSetDevice(ctx->device));
   Scratch s;
   double *ds = s.up(ctx->model.statd.data(), (size_t)x->S);
-  double *du = s.up<double>(nullptr, x->N), *dt = s.up<double>(nullptr, 2);
+  double *du = s.up<double>(nullptr, x->N), *dt = s.up<double>(nullptr, 1);
   CHECK(ds && du && dt, PP_ENOMEM, "device allocation failed");
-  hipLaunchKernelGGL(util_kernel, dim3((x->N + 255) / 256), dim3(256), 0, ctx->stream, du, ds, x->a, y->a, z->a,
-                     nullptr, 0, x->N, x->R, x->N, x->S);
-  hipLaunchKernelGGL(logsum_kernel, dim3(1), dim3(64), 0, ctx->stream, du, nullptr, 0, x->N, x->R, 1, dt);
-  hipLaunchKernelGGL(gv::finish_logdot_kernel, dim3(1), dim3(1), 0, ctx->stream, dt, x->e, y->e, z->e, nullptr, 0,
-                     x->N - 1, dt + 1);
-  return gv::fetch_double(ctx, dt + 1, out);
+  launch_logsum(ctx->stream, du, ds, x->a, y->a, z->a, nullptr, 0, x->N, x->R, x->N, x->S, 1, x->e, y->e, z->e, dt);
+  return gv::fetch_double(ctx, dt, out);
 }
 
 int pp_gmix_site_log_like_arr3(pp_ctx *ctx, const pp_glv *x, const pp_glv *y, const pp_glv *z, double *out) {

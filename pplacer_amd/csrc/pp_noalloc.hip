@@ -73,10 +73,8 @@ extern "C" int pp_ten_masked_logdot_noalloc(const double *x, const double *y, co
   const int st = scratch_of_current_device(&util);
   if (st) return st;
   hipStream_t s = static_cast<hipStream_t>(stream);
-  if (n_sites > 0)
-    hipLaunchKernelGGL(pp::util_kernel, dim3((n_sites + 255) / 256), dim3(256), 0, s, util, nullptr, x, y, nullptr,
-                       mask, 0, n_sites, n_rates, n_sites, n_states);
-  hipLaunchKernelGGL(pp::logsum_kernel, dim3(1), dim3(64), 0, s, util, mask, 0, n_sites, n_rates, 1, out);
+  pp::launch_logsum(s, util, nullptr, x, y, nullptr, mask, 0, n_sites, n_rates, n_sites, n_states, 1, nullptr, nullptr,
+                    nullptr, out);
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess) {
     pp::set_error(std::string("kernel launch failed: ") + hipGetErrorString(e));
