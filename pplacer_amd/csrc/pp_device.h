@@ -54,6 +54,26 @@ __device__ __forceinline__ double readlane_f64(double v, int l) {
 // stays known to be uniform.
 __device__ __forceinline__ bool wave_true(bool c) { return __builtin_amdgcn_ballot_w64(c) != 0; }
 
+// The lane index as a value the compiler cannot move out of a loop: what is
+// computed from it (LDS addresses above all) is made again where it is used
+// instead of being kept in registers across the probes.
+__device__ __forceinline__ int fresh_lane() {
+  int l = threadIdx.x & 63;
+  asm volatile("" : "+v"(l));
+  return l;
+}
+
+// The kernel's argument block (its only argument), to be read where a field is
+// used: what was read through an earlier pointer is not kept, so that the
+// control's loops do not hold two dozen pointers in scalar registers across
+// the probes.
+template <class Args>
+__device__ __forceinline__ const Args __attribute__((address_space(4))) *kernel_args() {
+  auto p = (const Args __attribute__((address_space(4))) *)__builtin_amdgcn_kernarg_segment_ptr();
+  asm volatile("" : "+s"(p));
+  return p;
+}
+
 // A wave-uniform double moved to scalar registers: for control values that
 // live long between uses, which then cost no vector register.
 __device__ __forceinline__ double scalar(double v) {

@@ -500,7 +500,7 @@ __device__ __forceinline__ void mw_worker_stream(char *smem, const MWLayout<Real
 // cap, too) and the lane's codes in `present`.
 __device__ __forceinline__ int mask_sites(const uint8_t *codes, int N, int n_inf, int cap, int *list,
                                           unsigned &present) {
-  const int lane = threadIdx.x & 63;
+  const int lane = fresh_lane();
   int total = 0;
   for (int k0 = 0; k0 < N; k0 += 512) {
     int c[8];
@@ -553,7 +553,6 @@ struct MWMaster : ThreeTaxControl<MWMaster<Real, R, SPL, CAT, STRICT>> {
   int lane, n_workers, cap_sites, n_codes, n_inf, n_sl;
   int n_amb;  // ambiguity codes present in the query
   double log_R;
-  double m_rate, m_l;  // the lane's rate and eigenvalue (tables)
 
   // cap: the longest masked length the launch takes (the layout's capacity)
   __device__ __forceinline__ void init(char *smem, const DevModel *dm, int cap) {
@@ -573,8 +572,6 @@ struct MWMaster : ThreeTaxControl<MWMaster<Real, R, SPL, CAT, STRICT>> {
     n_inf = dm->n_inf;
     log_R = dm->log_R;
     n_amb = 0;
-    m_rate = sh->rates[(lane >> 4) & (R - 1)];
-    m_l = sh->l[lane & 3];
     c_pend = c_dist = c_prox = __builtin_nan("");
   }
 
@@ -615,7 +612,7 @@ struct MWMaster : ThreeTaxControl<MWMaster<Real, R, SPL, CAT, STRICT>> {
   __device__ __forceinline__ void gather(int loc) {
     if (lane == 0) sh->loc = loc;
     command(CMD_GATHER);
-    const long long es = wave_sum_ll(lane < n_workers ? sh->ipart[lane] : 0);
+    const long long es = wave_sum_ll(fresh_lane() < n_workers ? sh->ipart[fresh_lane()] : 0);
     esum = scalar((double)es);
     c_dist = c_prox = __builtin_nan("");
     have_last = false;
@@ -640,7 +637,7 @@ struct MWMaster : ThreeTaxControl<MWMaster<Real, R, SPL, CAT, STRICT>> {
   __device__ __forceinline__ void ambiguity_rows(double p, bool active, Real *at) const {
     const double p0 = dpp_f64<0x00>(p), p1 = dpp_f64<0x55>(p), p2 = dpp_f64<0xAA>(p), p3 = dpp_f64<0xFF>(p);
     if (active)
-      for (int slot = 4 + (lane & 3); slot < 4 + n_amb; slot += 4) {
+      for (int slot = 4 + (fresh_lane() & 3); slot < 4 + n_amb; slot += 4) {
         const double *lv = sh->lv + sh->slot_code[slot] * 4;
         double acc = 0.0;
         acc = acc + p0 * lv[0];
@@ -655,6 +652,8 @@ struct MWMaster : ThreeTaxControl<MWMaster<Real, R, SPL, CAT, STRICT>> {
       cat_tables(new_pend, new_dist);
       return;
     }
+    const int lane = fresh_lane();
+    const double m_rate = sh->rates[(lane >> 4) & (R - 1)], m_l = sh->l[lane & 3];
     double mx[4], mxit[4];  // the lane's row of x and of xit
 #pragma unroll
     for (int k = 0; k < 4; k++) {
@@ -693,6 +692,8 @@ struct MWMaster : ThreeTaxControl<MWMaster<Real, R, SPL, CAT, STRICT>> {
   // j forms entry (i, j) of every fourth category's matrices, with its rows of
   // x and xit in registers, and the ambiguity rows from its quad.
   __device__ __forceinline__ void cat_exps(double bl, double *e) {
+    const int lane = fresh_lane();
+    const double m_l = sh->l[lane & 3];
     for (int t = lane; t < 4 * n_sl; t += 64) e[t] = texp((sh->rates[t >> 2] * bl) * m_l);
   }
   static __device__ __forceinline__ double cat_entry(const double *e, const double (&mx)[4], const double (&mxit)[4]) {
@@ -709,6 +710,7 @@ struct MWMaster : ThreeTaxControl<MWMaster<Real, R, SPL, CAT, STRICT>> {
     }
     if (new_pend) cat_exps(pend_bl, e2);
     wave_lds_sync();
+    const int lane = fresh_lane();
     double mx[4], mxit[4];
 #pragma unroll
     for (int k = 0; k < 4; k++) {
@@ -744,7 +746,7 @@ struct MWMaster : ThreeTaxControl<MWMaster<Real, R, SPL, CAT, STRICT>> {
     if constexpr (L::strict) {
       tot = wave_sequential_sum(slog, M);
     } else {
-      const double pv = sh->part[lane & 15];  // lane w: worker wave w's partial, added in wave order
+      const double pv = sh->part[fresh_lane() & 15];  // lane w: worker wave w's partial, added in wave order
       tot = readlane_f64(pv, 0);
       for (int w = 1; w < n_workers; w++) tot += readlane_f64(pv, w);
     }

@@ -405,6 +405,7 @@ struct ProtMaster : ThreeTaxControl<ProtMaster<Real, R>> {
 
   // The exponentials of Diagd.multi_exp for the changed branch lengths.
   __device__ __forceinline__ void tables(bool new_pend, bool new_dist) {
+    const int lane = fresh_lane();
     // one table per transition-matrix slice: rate (gamma) or category (CAT)
     if (new_dist) {
       for (int t = lane; t < 2 * n_sl * S; t += 64) {
@@ -431,7 +432,7 @@ struct ProtMaster : ThreeTaxControl<ProtMaster<Real, R>> {
       sh->tile_next = 0;
     }
     command(new_dist ? CMD_PROBE_DIST : CMD_PROBE);
-    const double pv = sh->part[lane & 15];  // lane w: worker wave w's partial, added in wave order
+    const double pv = sh->part[fresh_lane() & 15];  // lane w: worker wave w's partial, added in wave order
     double tot = readlane_f64(pv, 0);
     for (int w = 1; w < n_workers; w++) tot += readlane_f64(pv, w);
     c_pend = scalar(pend_bl);

@@ -117,7 +117,7 @@ __device__ __forceinline__ double wave_scan_f64(double v) {
 // starts up to l.  The steps of wave_scan_f64; a step's source is taken where
 // it lies in the lane's own run.
 __device__ __forceinline__ double wave_run_scan_f64(double v, unsigned long long starts) {
-  const int lane = threadIdx.x & 63;
+  const int lane = fresh_lane();
   const int first = 63 - __builtin_clzll(starts & (~0ull >> (63 - lane)));
   const int back = lane - first;  // lanes of the run before this one
   double t = dpp_f64_or0<0x111, 0xF>(v);
@@ -144,7 +144,7 @@ struct SeqSumBlock {
   int B;
   double x[CAP > 0 ? CAP : 1];
   __device__ __forceinline__ void load(const double *v0, int b) {
-    v = v0 + (int)(threadIdx.x & 63) * b;
+    v = v0 + fresh_lane() * b;
     B = b;
 #pragma unroll
     for (int j = 0; j < CAP; j++) x[j] = v[j < B ? j : 0];
@@ -181,7 +181,8 @@ __device__ __forceinline__ double wave_sequential_sum_of(const double *v, int n,
     top = fmax(top, x);
   });
   const double incl = wave_scan_f64(a);
-  const double p = (threadIdx.x & 63) ? start + (incl - a) : start;  // approximate partial sum before the block
+  const bool inner = fresh_lane() != 0;
+  const double p = inner ? start + (incl - a) : start;  // approximate partial sum before the block
   double Q = -(start + readlane_f64(incl, 63));
   if (wave_true(!(top <= 0.0))) {  // not every term is <= 0
     double q = 0.0;
@@ -197,7 +198,7 @@ __device__ __forceinline__ double wave_sequential_sum_of(const double *v, int n,
     tie |= fabs(x - (t - s)) == half_u;  // the addition's exact error, in a clean block
     s = t;
   });
-  const bool clean = ((threadIdx.x & 63) != 0) & (top <= 0.0) & (start <= 0.0) & !tie & (Q <= 0x1p+996) & (Q >= 0x1p-900) & (fabs(p) > delta) &
+  const bool clean = inner & (top <= 0.0) & (start <= 0.0) & !tie & (Q <= 0x1p+996) & (Q >= 0x1p-900) & (fabs(p) > delta) &
                      (__builtin_amdgcn_frexp_exp(fabs(p) - delta) == __builtin_amdgcn_frexp_exp(fabs(s) + delta));
   const unsigned long long again = __builtin_amdgcn_ballot_w64(!clean) | 1ull;
   const double move = wave_run_scan_f64(clean ? s - p : 0.0, again);

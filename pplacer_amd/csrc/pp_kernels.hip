@@ -185,15 +185,15 @@ __host__ __device__ __forceinline__ size_t taken_bytes(int E) { return (size_t)2
 struct NextEdge {
   const double *sc;
   unsigned *taken;
-  int E, lane;
+  int E;
   unsigned long long key;
   int edge;  // INT_MAX: the lane has none left
 
-  __device__ __forceinline__ void init(const double *scores, unsigned *flags, int n_edges, int lane_) {
+  __device__ __forceinline__ void init(const double *scores, unsigned *flags, int n_edges) {
+    const int lane = fresh_lane();
     sc = scores;
     taken = flags;
     E = n_edges;
-    lane = lane_;
     const int n_words = (int)(taken_bytes(E) / 256);
     for (int w = 0; w < n_words; w++) taken[w * 64 + lane] = 0u;
     key = ~0ull;
@@ -213,6 +213,7 @@ struct NextEdge {
   }
   // The next edge, marked taken; INT_MAX when none is left.
   __device__ __forceinline__ int take() {
+    const int lane = fresh_lane();
     unsigned long long bk = key;
     int bi = edge;
     wave_argmin(bk, bi);
@@ -240,35 +241,38 @@ struct NextEdge {
 
 // Baseball over one work queue of queries, for either engine's master.
 template <class Master>
-__device__ __forceinline__ void pitch_loop(const PitchArgs &a, Master &m, unsigned *taken) {
+__device__ __forceinline__ void pitch_loop(Master &m, unsigned *taken) {
   const int lane = m.lane;
   for (;;) {
+    const auto a = kernel_args<PitchArgs>();
     int qi = 0;
-    if (lane == 0) qi = atomicAdd(a.counter, 1);
+    if (lane == 0) qi = atomicAdd(a->counter, 1);
     qi = __builtin_amdgcn_readfirstlane(qi);  // wave-uniform: branches below hold barriers
-    if (qi >= a.nq) break;
-    const int q = a.qlist[qi];
-    const int M = m.load_query(a.codes + (size_t)q * a.N, a.N, q);
+    if (qi >= a->nq) break;
+    const int q = a->qlist[qi];
+    const int M = m.load_query(a->codes + (size_t)q * a->N, a->N, q);
     if (M == 0 || M > m.cap_sites) {
-      if (lane == 0) { a.n_res[q] = 0; a.status[q] = M == 0 ? PP_Q_NO_INFORMATIVE : PP_Q_RANK_EXHAUSTED; }
+      if (lane == 0) { a->n_res[q] = 0; a->status[q] = M == 0 ? PP_Q_NO_INFORMATIVE : PP_Q_RANK_EXHAUSTED; }
       continue;
     }
     NextEdge next;
-    next.init(a.scores + (size_t)q * a.E, taken, a.E, lane);
+    next.init(a->scores + (size_t)q * a->E, taken, a->E);
     double like_record = -INFINITY;
     long long n_strikes = 0, calls = 0, probes = 0, dprobes = 0;
     int n_res = 0, status = PP_Q_OK;
     for (;;) {
+      const auto a = kernel_args<PitchArgs>();
       const int loc = next.take();
       if (loc == INT_MAX) break;
       m.gather(loc);
-      const double cut = a.bl[loc];
-      m.set_state(cut, a.start_pend, cut / 2.);
+      const double cut = a->bl[loc];
+      m.set_state(cut, a->start_pend, cut / 2.);
       m.n_calls = 0;
       m.n_probes = 0;
       m.n_dist_probes = 0;
       double ll, pend, dist;
-      const int st = m.safe_optimize(a.initial_tol, a.max_pend, a.start_pend, cut, &ll, &pend, &dist);
+      const int st = m.safe_optimize(a->initial_tol, a->max_pend, a->start_pend, cut, &ll, &pend, &dist);
+      const auto b = kernel_args<PitchArgs>();
       calls += m.n_calls;
       probes += m.n_probes;
       dprobes += m.n_dist_probes;
@@ -281,27 +285,28 @@ __device__ __forceinline__ void pitch_loop(const PitchArgs &a, Master &m, unsign
       if (lane == 0) {
         Res r;
         r.ll = ll; r.pend = pend; r.dist = dist; r.loc = loc; r.flags = st == ST_MAXITER;
-        a.res[(size_t)q * a.cap + n_res] = r;
+        b->res[(size_t)q * b->cap + n_res] = r;
       }
       const int prev_len = n_res;
       n_res++;
-      if (prev_len >= a.t_max_pitches) break;
+      if (prev_len >= b->t_max_pitches) break;
       else if (wave_true(ll > like_record)) like_record = scalar(ll);
-      else if (wave_true(ll < like_record - a.strike_box)) {
-        if (n_strikes + 1 >= a.t_max_strikes) break;
+      else if (wave_true(ll < like_record - b->strike_box)) {
+        if (n_strikes + 1 >= b->t_max_strikes) break;
         n_strikes++;
       }
-      if (n_res >= a.cap) break;
+      if (n_res >= b->cap) break;
     }
+    const auto b = kernel_args<PitchArgs>();
     if (lane == 0) {
-      a.n_res[q] = n_res;
-      a.status[q] = (status == PP_Q_OK && n_res == 0) ? PP_Q_NO_RESULTS : status;
-      atomicAdd(a.n_calls, (unsigned long long)calls);
-      atomicAdd(a.n_pitched, (unsigned long long)n_res);
-      atomicAdd(a.n_calls + 2, (unsigned long long)((probes - dprobes) * M));
-      atomicAdd(a.n_calls + 3, (unsigned long long)(dprobes * M));
-      atomicAdd(a.n_calls + 4, (unsigned long long)((probes - dprobes) * M));
-      atomicAdd(a.n_calls + 5, (unsigned long long)(dprobes * M));
+      b->n_res[q] = n_res;
+      b->status[q] = (status == PP_Q_OK && n_res == 0) ? PP_Q_NO_RESULTS : status;
+      atomicAdd(b->n_calls, (unsigned long long)calls);
+      atomicAdd(b->n_pitched, (unsigned long long)n_res);
+      atomicAdd(b->n_calls + 2, (unsigned long long)((probes - dprobes) * M));
+      atomicAdd(b->n_calls + 3, (unsigned long long)(dprobes * M));
+      atomicAdd(b->n_calls + 4, (unsigned long long)((probes - dprobes) * M));
+      atomicAdd(b->n_calls + 5, (unsigned long long)(dprobes * M));
     }
   }
   m.command(CMD_EXIT);
@@ -362,7 +367,7 @@ void pitch_mw_kernel(PitchArgs a) {
   }
   MWMaster<Real, R, SPL, CAT, STRICT> m;
   m.init(smem, a.model, cap);
-  pitch_loop(a, m, taken);
+  pitch_loop(m, taken);
 }
 
 // The 20-state workers of either form: FP64 in the eigenbasis
@@ -418,69 +423,71 @@ void pitch_prot_kernel(PitchArgs a) {
   }
   ProtMaster<Real, R> m;
   m.init(smem, a.model, a.cap_pairs);
-  pitch_loop(a, m, taken);
+  pitch_loop(m, taken);
 }
 
 // Three_tax.optimize jobs of one work queue, for either engine's master.
 template <class Master>
-__device__ __forceinline__ void optimize_loop(const OptArgs &a, Master &m) {
+__device__ __forceinline__ void optimize_loop(Master &m) {
   const int lane = m.lane;
   for (;;) {
+    const auto a = kernel_args<OptArgs>();
     int job = 0;
-    if (lane == 0) job = atomicAdd(a.counter, 1);
+    if (lane == 0) job = atomicAdd(a->counter, 1);
     job = __builtin_amdgcn_readfirstlane(job);
-    if (job >= a.n_jobs) break;
+    if (job >= a->n_jobs) break;
     int q, loc;
     double pend0, dist0;
     Res *slot = nullptr;
     int jj = 0;
-    if (a.mode == 1) {
-      const int qi = job / a.K, k = job % a.K;
-      q = a.qlist[qi];
-      if (k >= a.n_keep[q]) continue;
-      slot = a.kept + (size_t)q * a.K + k;
+    if (a->mode == 1) {
+      const int qi = job / a->K, k = job % a->K;
+      q = a->qlist[qi];
+      if (k >= a->n_keep[q]) continue;
+      slot = a->kept + (size_t)q * a->K + k;
       loc = slot->loc;
       pend0 = slot->pend;
       dist0 = slot->dist;
     } else {
-      jj = a.qlist ? a.qlist[job] : job;
-      q = a.job_q[jj];
-      loc = a.job_loc[jj];
-      pend0 = a.job_pend[jj];
-      dist0 = a.job_dist[jj];
+      jj = a->qlist ? a->qlist[job] : job;
+      q = a->job_q[jj];
+      loc = a->job_loc[jj];
+      pend0 = a->job_pend[jj];
+      dist0 = a->job_dist[jj];
     }
-    const int M = m.load_query(a.codes + (size_t)q * a.N, a.N, q);
+    const int M = m.load_query(a->codes + (size_t)q * a->N, a->N, q);
     if (M == 0 || M > m.cap_sites) {
-      if (lane == 0 && a.mode == 0) a.out_status[jj] = M == 0 ? PP_Q_NO_INFORMATIVE : PP_Q_RANK_EXHAUSTED;
+      if (lane == 0 && a->mode == 0) a->out_status[jj] = M == 0 ? PP_Q_NO_INFORMATIVE : PP_Q_RANK_EXHAUSTED;
       continue;
     }
     m.gather(loc);
-    const double cut = a.bl[loc];
+    const double cut = a->bl[loc];
     m.set_state(cut, pend0, dist0);
     m.n_calls = 0;
     m.n_probes = 0;
     m.n_dist_probes = 0;
     double ll, pend, dist;
-    const int st = m.safe_optimize(a.tol, a.max_pend, a.start_pend, cut, &ll, &pend, &dist);
+    const int st = m.safe_optimize(a->tol, a->max_pend, a->start_pend, cut, &ll, &pend, &dist);
+    const auto b = kernel_args<OptArgs>();
     if (lane == 0) {
-      atomicAdd(a.n_calls, (unsigned long long)m.n_calls);
-      atomicAdd(a.n_calls + 2, (unsigned long long)((m.n_probes - m.n_dist_probes) * M));
-      atomicAdd(a.n_calls + 3, (unsigned long long)(m.n_dist_probes * M));
-      if (a.mode == 1) {
+      atomicAdd(b->n_calls, (unsigned long long)m.n_calls);
+      atomicAdd(b->n_calls + 2, (unsigned long long)((m.n_probes - m.n_dist_probes) * M));
+      atomicAdd(b->n_calls + 3, (unsigned long long)(m.n_dist_probes * M));
+      if (b->mode == 1) {
         if (st == ST_OK || st == ST_MAXITER) {
           slot->ll = ll;
           slot->pend = pend;
           slot->dist = dist;
         } else if (!is_gsl(st)) {
-          a.status[q] = st == ST_FIND_START ? PP_Q_FIND_START
+          b->status[q] = st == ST_FIND_START ? PP_Q_FIND_START
                         : st == ST_INVALID_START ? PP_Q_INVALID_START : PP_Q_ASSERT;
         }  // a GSL problem in the final optimisation keeps the initial result
       } else {
-        a.out_ll[jj] = ll;
-        a.out_pend[jj] = pend;
-        a.out_dist[jj] = dist;
-        a.out_calls[jj] = (int)m.n_calls;
-        a.out_status[jj] = st;
+        b->out_ll[jj] = ll;
+        b->out_pend[jj] = pend;
+        b->out_dist[jj] = dist;
+        b->out_calls[jj] = (int)m.n_calls;
+        b->out_status[jj] = st;
       }
     }
   }
@@ -491,62 +498,64 @@ __device__ __forceinline__ void optimize_loop(const OptArgs &a, Master &m) {
 // or per job (mode 0), Three_tax.calc_marg_prob from the placement's branch
 // lengths with the prior of its edge.  FP64 only, as the final likelihoods.
 template <class Master>
-__device__ __forceinline__ void marginal_loop(const OptArgs &a, Master &m) {
+__device__ __forceinline__ void marginal_loop(Master &m) {
   const int lane = m.lane;
 #pragma unroll 1
   for (;;) {
+    const auto a = kernel_args<OptArgs>();
     int job = 0;
-    if (lane == 0) job = atomicAdd(a.counter, 1);
+    if (lane == 0) job = atomicAdd(a->counter, 1);
     job = __builtin_amdgcn_readfirstlane(job);
-    if (job >= a.n_jobs) break;
+    if (job >= a->n_jobs) break;
     int q, loc;
     double pend0, dist0;
     Res *slot = nullptr;
     int jj = 0;
-    if (a.mode == 1) {
-      const int qi = job / a.K, k = job % a.K;
-      q = a.qlist[qi];
-      if (a.status[q] != PP_Q_OK || k >= a.n_keep[q]) continue;
-      slot = a.kept + (size_t)q * a.K + k;
+    if (a->mode == 1) {
+      const int qi = job / a->K, k = job % a->K;
+      q = a->qlist[qi];
+      if (a->status[q] != PP_Q_OK || k >= a->n_keep[q]) continue;
+      slot = a->kept + (size_t)q * a->K + k;
       loc = slot->loc;
       pend0 = slot->pend;
       dist0 = slot->dist;
     } else {
-      jj = a.qlist ? a.qlist[job] : job;
-      q = a.job_q[jj];
-      loc = a.job_loc[jj];
-      pend0 = a.job_pend[jj];
-      dist0 = a.job_dist[jj];
+      jj = a->qlist ? a->qlist[job] : job;
+      q = a->job_q[jj];
+      loc = a->job_loc[jj];
+      pend0 = a->job_pend[jj];
+      dist0 = a->job_dist[jj];
     }
-    const int M = m.load_query(a.codes + (size_t)q * a.N, a.N, q);
+    const int M = m.load_query(a->codes + (size_t)q * a->N, a->N, q);
     if (M == 0 || M > m.cap_sites) {
-      if (lane == 0 && a.mode == 0) a.out_status[jj] = M == 0 ? PP_Q_NO_INFORMATIVE : PP_Q_RANK_EXHAUSTED;
+      if (lane == 0 && a->mode == 0) a->out_status[jj] = M == 0 ? PP_Q_NO_INFORMATIVE : PP_Q_RANK_EXHAUSTED;
       continue;
     }
     m.gather(loc);
-    m.set_state(a.bl[loc], pend0, dist0);  // tt_edges_from_placement (core.ml:241-250)
-    m.pr_kind = a.prior_kind;
-    m.pr_mu = a.prior_mean[loc];
+    m.set_state(a->bl[loc], pend0, dist0);  // tt_edges_from_placement (core.ml:241-250)
+    m.pr_kind = a->prior_kind;
+    m.pr_mu = a->prior_mean[loc];
     m.n_calls = 0;
     m.n_probes = 0;
     m.n_dist_probes = 0;
     double marg = 0.;
-    const int st = m.calc_marg_prob(a.pp_rel_err, a.max_pend, &marg);
+    const int st = m.calc_marg_prob(a->pp_rel_err, a->max_pend, &marg);
+    const auto b = kernel_args<OptArgs>();
     if (lane == 0) {
-      atomicAdd(a.n_calls, (unsigned long long)m.n_calls);
-      atomicAdd(a.n_calls + 2, (unsigned long long)((m.n_probes - m.n_dist_probes) * M));
-      atomicAdd(a.n_calls + 3, (unsigned long long)(m.n_dist_probes * M));
-      if (a.mode == 1) {
+      atomicAdd(b->n_calls, (unsigned long long)m.n_calls);
+      atomicAdd(b->n_calls + 2, (unsigned long long)((m.n_probes - m.n_dist_probes) * M));
+      atomicAdd(b->n_calls + 3, (unsigned long long)(m.n_dist_probes * M));
+      if (b->mode == 1) {
         if (st == ST_OK) slot->marg = marg;
         else  // uncaught in the reference: the query fails
-          a.status[q] = st == ST_MAXITER ? PP_Q_MAXITER
+          b->status[q] = st == ST_MAXITER ? PP_Q_MAXITER
                         : st == ST_FIND_START ? PP_Q_FIND_START
                         : st == ST_INVALID_START ? PP_Q_INVALID_START
                         : st == ST_ASSERT ? PP_Q_ASSERT : PP_Q_GSL;
       } else {
-        a.out_ll[jj] = marg;
-        a.out_calls[jj] = (int)m.n_calls;
-        a.out_status[jj] = st;
+        b->out_ll[jj] = marg;
+        b->out_calls[jj] = (int)m.n_calls;
+        b->out_status[jj] = st;
       }
     }
   }
@@ -569,7 +578,7 @@ void optimize_mw_kernel(OptArgs a) {
   }
   MWMaster<Real, R, SPL, CAT, STRICT> m;
   m.init(smem, a.model, cap);
-  optimize_loop(a, m);
+  optimize_loop(m);
 }
 
 template <typename Real, int R>
@@ -583,7 +592,7 @@ void optimize_prot_kernel(OptArgs a) {
   }
   ProtMaster<Real, R> m;
   m.init(smem, a.model, a.cap_pairs);
-  optimize_loop(a, m);
+  optimize_loop(m);
 }
 
 template <int R, int MAXBD, int SPL, bool CAT, bool STRICT>
@@ -602,7 +611,7 @@ void marginal_mw_kernel(OptArgs a) {
   }
   MWMaster<double, R, SPL, CAT, STRICT> m;
   m.init(smem, a.model, cap);
-  marginal_loop(a, m);
+  marginal_loop(m);
 }
 
 template <int R>
@@ -616,7 +625,7 @@ __global__ __launch_bounds__(512) void marginal_prot_kernel(OptArgs a) {
   }
   ProtMaster<double, R> m;
   m.init(smem, a.model, a.cap_pairs);
-  marginal_loop(a, m);
+  marginal_loop(m);
 }
 
 // ---------------------------------------------------------------------------
