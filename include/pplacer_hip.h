@@ -333,8 +333,10 @@ int pp_synchronize(pp_ctx *ctx);
  *   pitch_streams[f], refine_streams[f]: streams over which the 4-state
  *     baseball phase and the refinement phase spread their masked-length
  *     buckets, for form f (0 = PP_FP64, 1 = PP_FP32); 0 runs them one after
- *     another on the main stream; at most PP_MAX_BUCKET_STREAMS.  The -p
- *     phase and 20-state passes always run on the main stream.
+ *     another on the main stream; at most PP_MAX_BUCKET_STREAMS.  Until a
+ *     shape is set, passes in chunks of at most 32,768 queries spread the
+ *     baseball and -p phases over at least 4 streams; after that the -p phase
+ *     runs on the main stream, as 20-state passes always do.
  *   chunk: queries per device chunk (stage 1 of the next chunk overlaps
  *     stage 2 of the current one), 1 .. PP_MAX_CHUNK, further capped so that a
  *     chunk's scores ([chunk][n_edges] doubles) stay under 2 GiB.

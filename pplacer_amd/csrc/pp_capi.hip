@@ -55,6 +55,18 @@ static_assert(kChunk <= PP_MAX_CHUNK, "default chunk out of range");
 // 2,000 taxa.
 constexpr int kPitchStreams[2] = {0, 8};
 constexpr int kRefineStreams[2] = {4, 4};
+// Until a launch shape is given (pp_launch_config_set), 4-state passes of
+// chunks of at most kForkQueries run their baseball and -p phases over at least
+// kForkStreams streams: a bucket's launch is then a few rounds of the work
+// queue at most, and ends on a tail of a few long queries that the other
+// buckets fill.  FP64, main stream -> 4 streams, by queries: 16S reads on 2,000
+// taxa 2,000: 19.9 -> 15.9 ms, 10,000: 61.5 -> 54.6, 20,000: 140 -> 126,
+// 40,000: 235 -> 231, 80,000: 465 -> 460; Price-CAT 500: 18.7 -> 8.1, 8,000:
+// 63.7 -> 54.7, 30,000: 200 -> 185; full-length reads 257: 25.2 -> 14.5,
+// 5,000: 121 -> 110; with -p 100: 37.5 -> 15.1, 400: 40.4 -> 17.8, 8,000: 169
+// -> 149.  Larger chunks gain 2% at most and stay on the main stream, where a
+// launch's duration is the kernel's own.
+constexpr int kForkQueries = 32768, kForkStreams = 4;
 constexpr int kProtBlock = 512;   // lanes of a 20-state stage-2 workgroup (master + workers)
 
 struct DBuf {
@@ -96,6 +108,7 @@ struct pp_ctx {
   hipStream_t s1 = nullptr;           // stage 1 of the next chunk
   hipStream_t bs[kBucketStreams] = {};  // concurrent stage-2 buckets
   hipStream_t cur = nullptr;          // the stream the launch helpers use
+  bool launch_given = false;          // pp_launch_config_set has been called
   pp_launch_config launch{{kPitchStreams[0], kPitchStreams[1]}, {kRefineStreams[0], kRefineStreams[1]}, kChunk, 0};
   // graph mode: captured chunk loops by plan key (most recent last; a pass
   // and the FP64 re-placement of its FP32 failures keep one each)
@@ -1129,7 +1142,8 @@ int place_pass(pp_ctx *c, const pp_prefs *prefs, int precision, pp_stats *stats)
   LaunchStream ls(c, c->stream);
   const bool fp32 = precision == PP_FP32;
   const bool s2_fp32 = fp32 && stage2_fp32_ok(c);
-  // Concurrent buckets, measured at 100,000 queries: the FP32 form 323 -> 274
+  // Concurrent buckets (a short chunk's: kForkQueries), measured at 100,000
+  // queries: the FP32 form 323 -> 274
   // ms per pass with 4 streams, 258 -> 251 ms with 8 for its baseball; the
   // refinement with 4 streams (FP64 364 -> 356 ms; with 50,000-query chunks
   // the FP32 form's 273-279 ms with 8 -> 267-270 ms with 4).  The FP64
@@ -1137,7 +1151,11 @@ int place_pass(pp_ctx *c, const pp_prefs *prefs, int precision, pp_stats *stats)
   // launch's duration is the kernel's own (4 streams measured within 1% at
   // 50,000-query chunks), and a tuner may set them.  The 20-state kernels
   // share one scratch buffer and do not fork.
-  const int pitch_streams = c->model.S == 4 ? c->launch.pitch_streams[s2_fp32 ? 1 : 0] : 0;
+  const bool fork = c->model.S == 4 && !c->launch_given && Q <= (int64_t)kForkQueries * n_chunks;
+  const int pitch_streams = c->model.S != 4 ? 0
+                            : fork ? std::max(c->launch.pitch_streams[s2_fp32], kForkStreams)
+                                   : c->launch.pitch_streams[s2_fp32];
+  const int marg_streams = fork ? kForkStreams : 0;
   const int refine_streams = c->model.S == 4 ? c->launch.refine_streams[s2_fp32 ? 1 : 0] : 0;
   hipEvent_t e_t0 = pool.get(), e_t1 = pool.get();
   CHECK(e_t0 && e_t1, PP_EDEVICE, "hipEventCreate failed");
@@ -1402,9 +1420,7 @@ int place_pass(pp_ctx *c, const pp_prefs *prefs, int precision, pp_stats *stats)
       if (st) return st;
       if (!graph) HIPCHECK(hipEventRecord(mk.r1, c->stream));
       if (prefs->calc_pp) {  // core.ml:378-392, one job per kept placement
-        // on the main stream: forked over the refinement's streams, this phase
-        // measured 196 -> 215-221 ms (FP64) at 20,000 queries
-        st = phase(boff, 0, [&](int b) -> int {
+        st = phase(boff, marg_streams, [&](int b) -> int {
           OptArgs o = marg_proto;
           o.model = c->d_model;
           o.codes = codes;
@@ -1903,6 +1919,7 @@ int pp_launch_config_set(pp_ctx *c, const pp_launch_config *cfg) {
   CHECK(cfg->chunk >= 1 && cfg->chunk <= PP_MAX_CHUNK, PP_EINVAL, "chunk must be in 1..PP_MAX_CHUNK");
   CHECK(cfg->graph == 0 || cfg->graph == 1, PP_EINVAL, "graph must be 0 or 1");
   c->launch = *cfg;
+  c->launch_given = true;
   return PP_OK;
 }
 

@@ -317,7 +317,9 @@ class Placer:
     def launch_config(self) -> dict:
         """The pass's launch shape: streams per stage-2 phase and form
         (index 0 = FP64, 1 = FP32), queries per device chunk, and whether the
-        pass's launches are captured into a replayed HIP graph."""
+        pass's launches are captured into a replayed HIP graph.  Until a shape
+        is set, passes in short chunks use more streams than this says
+        (include/pplacer_hip.h, pp_launch_config)."""
         cfg = LaunchConfig()
         check(lib().pp_launch_config_get(self._ctx, C.byref(cfg)), "launch_config_get")
         return {"pitch_streams": list(cfg.pitch_streams), "refine_streams": list(cfg.refine_streams),
