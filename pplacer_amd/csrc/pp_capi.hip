@@ -1089,6 +1089,31 @@ struct LaunchStream {
 // finalize) runs chunk after chunk on the main stream; in the 4-state form a
 // phase's buckets can run concurrently on up to kBucketStreams streams (the
 // tails of their work queues overlap), joined before the next phase.
+// Short passes (kForkQueries): moves a chunk's queries of shorter masked-length
+// classes into the next longer class's launch while that holds at most two
+// rounds of the workgroups of its size that the device runs at once (4 waves
+// per SIMD).  Such launches last as long as their slowest query, and not all
+// of them run at once (streams share hardware queues): one launch of 400 reads
+// with -p took 4.1 ms for the baseball phase where six over 4 streams took
+// 10.4, and the pass 17.9 -> 11.8 ms; 257 full-length reads 14.6 -> 11.7,
+// 10,000 16S reads 55 -> 52; 2,000 Price-CAT reads 16.4 -> 15.0-16.5 (17.8
+// with one round, 18.5-19.6 with four).  A workgroup's spare waves hold no
+// sites and add 0.0 to a sum, so results do not depend on the launch; only
+// the one-rate FP32 baseball places its sites by the block size, and is left.
+void merge_buckets(const pp_ctx *c, std::vector<std::vector<int>> &buckets, bool fp32) {
+  for (int top = kLongBucket - 1; top > 0;) {
+    const int spl = spl_for(true, top);
+    const size_t room = (size_t)2 * c->n_cu * (1024 / block_for(top, spl));
+    int b = top - 1;
+    if (!buckets[top].empty() && (!fp32 || c->model.R == 4))
+      for (; b >= 0 && spl_for(true, b) == spl && buckets[top].size() + buckets[b].size() <= room; b--) {
+        buckets[top].insert(buckets[top].end(), buckets[b].begin(), buckets[b].end());
+        buckets[b].clear();
+      }
+    top = b;
+  }
+}
+
 int place_pass(pp_ctx *c, const pp_prefs *prefs, int precision, pp_stats *stats) {
   CHECK(prefs, PP_EINVAL, "prefs is null");
   CHECK(precision == PP_FP64 || precision == PP_FP32, PP_EINVAL, "precision must be PP_FP64 or PP_FP32");
@@ -1184,6 +1209,7 @@ int place_pass(pp_ctx *c, const pp_prefs *prefs, int precision, pp_stats *stats)
     if (c->model.S == 20)
       std::stable_sort(buckets[0].begin(), buckets[0].end(),
                        [&](int x, int y) { return c->qM[q0 + x] > c->qM[q0 + y]; });
+    if (fork) merge_buckets(c, buckets, s2_fp32);
     std::vector<int> &boff = boffs[ci];
     int n = 0;
     for (int b = 0; b < kBuckets; b++) {
