@@ -527,9 +527,9 @@ __device__ __forceinline__ int mask_sites(const uint8_t *codes, int N, int n_inf
 // ---------------------------------------------------------------------------
 // master wave
 // ---------------------------------------------------------------------------
-template <typename Real, int R, int SPL, bool CAT, bool STRICT>
-struct MWMaster : ThreeTaxControl<MWMaster<Real, R, SPL, CAT, STRICT>> {
-  using Ctl = ThreeTaxControl<MWMaster<Real, R, SPL, CAT, STRICT>>;
+template <typename Real, int R, int MAXBD, int SPL, bool CAT, bool STRICT>
+struct MWMaster : ThreeTaxControl<MWMaster<Real, R, MAXBD, SPL, CAT, STRICT>> {
+  using Ctl = ThreeTaxControl<MWMaster<Real, R, MAXBD, SPL, CAT, STRICT>>;
   using Ctl::M;
   using Ctl::pend_bl;
   using Ctl::dist_bl;
@@ -744,7 +744,7 @@ struct MWMaster : ThreeTaxControl<MWMaster<Real, R, SPL, CAT, STRICT>> {
     command(new_dist ? CMD_PROBE_DIST : CMD_PROBE);
     double tot;
     if constexpr (L::strict) {
-      tot = wave_sequential_sum(slog, M);
+      tot = wave_sequential_sum<SPL == 0 ? INT_MAX : SPL * (MAXBD - 64)>(slog, M);
     } else {
       const double pv = sh->part[fresh_lane() & 15];  // lane w: worker wave w's partial, added in wave order
       tot = readlane_f64(pv, 0);

@@ -10,8 +10,8 @@
 // on s_{k-1}).  A run of such additions moves any starting value of the
 // binade by the same multiple of u_E.
 //
-// So the terms are split into 64 contiguous blocks of B = ceil(n / 64), one a
-// lane, and
+// So every lane adds the first 32 terms one by one, and the others are split
+// into 64 contiguous blocks, one a lane, of 4, 8, 16 or 24 terms:
 //  1. a DPP scan of block sums gives each lane an approximate partial sum p
 //     before its block, within delta = (4n + 256) 2^-53 sum|v| of the true one
 //     (recursive summation error bounds, doubled);
@@ -24,18 +24,22 @@
 //     u_E, less than 2^53 of them), in any order: a DPP scan that restarts at
 //     the other blocks;
 //  4. the other blocks (the first, those that change the binade or hold a
-//     tie; about 8 at 300 terms) are run again in order from the true sum.
+//     tie; about 5 at 300 terms) are run again in order from the true sum.
 //     Whatever a block holds (mixed signs, infinities, NaN), that is the
 //     sequential sum itself, so only how many blocks are run again depends on
 //     the terms.
 //
-// What it costs: B dependent additions twice, two scans of 6 steps, and B
-// additions and two lane reads for each block run again.  On one wave: 1,700
-// cycles at 300 terms against 5,200 for the chain of one lane (17 cycles a
-// term), 1,000 against 1,900 at 100.
+// What bounds it is the length of the dependent chain (an FP64 addition 8
+// cycles, a lane read into the next addition 32): two scans of 6 steps, the
+// blocks' additions twice and again for each block run again.  In the engine's
+// control wave: 2,150 cycles at 209 terms and 4,430 at 1,080 beside another
+// workgroup; 2,790 and 10,280 without the head, with blocks of ceil(n / 64)
+// terms read from LDS beyond 512; 17 cycles a term for the chain of one lane.
 #pragma once
 
 #include <hip/hip_runtime.h>
+
+#include <climits>
 
 #include "pp_device.h"
 
@@ -43,6 +47,7 @@ namespace pp {
 
 // Longest sum the wave takes; longer ones go to the one-lane chain.
 constexpr int kSeqSumWaveMax = 4096;
+constexpr int kSeqSumHead = 32;
 
 // s + v[0] + v[1] + ... + v[n-1], one lane.  A dependent chain, so it is fed
 // from LDS two blocks of eight ahead: the loads of one block are in flight
@@ -79,7 +84,9 @@ __device__ __forceinline__ double ordered_sum(const double *v, int n, double s =
 // source lane falls outside the row, get 0.
 template <int CTRL, int ROWMASK>
 __device__ __forceinline__ int dpp_i32_or0(int v) {
-  return __builtin_amdgcn_update_dpp(0, v, CTRL, ROWMASK, 0xF, false);
+  // with whole rows the hardware's own zero for a source outside the row
+  // (bound_ctrl) saves setting the result first
+  return __builtin_amdgcn_update_dpp(0, v, CTRL, ROWMASK, 0xF, ROWMASK == 0xF);
 }
 template <int CTRL, int ROWMASK>
 __device__ __forceinline__ double dpp_f64_or0(double v) {
@@ -102,13 +109,23 @@ __device__ __forceinline__ int wave_scan_i32(int v) {
   v += dpp_i32_or0<0x143, 0xC>(v);
   return v;
 }
-__device__ __forceinline__ double wave_scan_f64(double v) {
+// between(): called before and after each of the six steps, for work that the
+// steps' latency covers.
+template <class F>
+__device__ __forceinline__ double wave_scan_f64(double v, F &&between) {
+  between();
   v += dpp_f64_or0<0x111, 0xF>(v);
+  between();
   v += dpp_f64_or0<0x112, 0xF>(v);
+  between();
   v += dpp_f64_or0<0x114, 0xF>(v);
+  between();
   v += dpp_f64_or0<0x118, 0xF>(v);
+  between();
   v += dpp_f64_or0<0x142, 0xA>(v);
+  between();
   v += dpp_f64_or0<0x143, 0xC>(v);
+  between();
   return v;
 }
 
@@ -135,70 +152,104 @@ __device__ __forceinline__ double wave_run_scan_f64(double v, unsigned long long
   return v;
 }
 
-// The terms of a lane's block, B (wave-uniform) of them from v + lane B: in
-// registers when the block has at most CAP, else read from LDS as they are
-// needed.
+// The terms of a lane's block: CAP of them from v + first, in registers, 0.0
+// for a lane past the terms; CAP = 0: B (wave-uniform) of them, read from LDS
+// as they are needed.
 template <int CAP>
 struct SeqSumBlock {
-  const double *v;
-  int B;
   double x[CAP > 0 ? CAP : 1];
-  __device__ __forceinline__ void load(const double *v0, int b) {
-    v = v0 + fresh_lane() * b;
-    B = b;
+  const double *v;
+  int B, rest;  // CAP = 0: terms from v
+  __device__ __forceinline__ void load(const double *terms, int n) {
+    if constexpr (CAP > 0) {
+      const int at = fresh_lane() * CAP;
 #pragma unroll
-    for (int j = 0; j < CAP; j++) x[j] = v[j < B ? j : 0];
+      for (int j = 0; j < CAP; j++) x[j] = 0.0;
+      if (at < n)
+#pragma unroll
+        for (int j = 0; j < CAP; j++) x[j] = terms[at + j];
+    } else {
+      B = (n + 63) >> 6;
+      v = terms + fresh_lane() * B;
+      rest = n - fresh_lane() * B;
+    }
   }
   template <class F>
   __device__ __forceinline__ void each(F &&f) const {
     if constexpr (CAP > 0) {
 #pragma unroll
-      for (int j = 0; j < CAP; j++)
-        if (j < B) f(x[j]);
+      for (int j = 0; j < CAP; j++) f(x[j]);
     } else {
-      int j = 0;
 #pragma unroll 1
-      for (; j + 8 <= B; j += 8) {
+      for (int j = 0; j < B; j += 8) {
         double y[8];
 #pragma unroll
-        for (int i = 0; i < 8; i++) y[i] = v[j + i];
+        for (int i = 0; i < 8; i++) y[i] = j + i < B && j + i < rest ? v[j + i] : 0.0;
 #pragma unroll
         for (int i = 0; i < 8; i++) f(y[i]);
       }
-#pragma unroll 1
-      for (; j < B; j++) f(v[j]);
     }
   }
 };
 
+// head: the first terms, a multiple of 8, that every lane adds one by one.
+// They hold about half of the binade changes and ties, and their chain runs in
+// the shadow of the scan.
 template <int CAP>
-__device__ __forceinline__ double wave_sequential_sum_of(const double *v, int n, int B, int *n_events, double start) {
+__device__ __forceinline__ double wave_sequential_sum_of(const double *v, int head, int n, int *n_events,
+                                                         double start) {
   SeqSumBlock<CAP> blk;
-  blk.load(v, B);
-  double a = 0.0, top = -INFINITY;
+  blk.load(v + head, n - head);
+  // The head's loads eight ahead, its additions among those of the blocks and the
+  // scan's steps, as written (left to itself the compiler finished the scan
+  // first and then waited for LDS at every eighth addition)
+  double h = start, y[8];
+#pragma unroll
+  for (int j = 0; j < 8; j++) y[j] = v[j];
+  blk.load(v + head, n - head);
+  double a = 0.0;
+  double top = 0.0;
   blk.each([&](double x) {
     a += x;
     top = fmax(top, x);
   });
-  const double incl = wave_scan_f64(a);
+  const bool neg = top <= 0.0;
+  int i = 0;
+  const double incl = wave_scan_f64(a, [&] {
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int j = 0; j < 5; j++, i++)
+      if (i < kSeqSumHead) {
+        h += y[i % 8];
+        if (i + 8 < kSeqSumHead) y[i % 8] = v[i + 8];
+      }
+    __builtin_amdgcn_sched_barrier(0);
+  });
+#pragma unroll 1
+  for (int k = kSeqSumHead; k < head; k += 8) {
+#pragma unroll
+    for (int j = 0; j < 8; j++) y[j] = v[k + j];
+#pragma unroll
+    for (int j = 0; j < 8; j++) h += y[j];
+  }
   const bool inner = fresh_lane() != 0;
-  const double p = inner ? start + (incl - a) : start;  // approximate partial sum before the block
-  double Q = -(start + readlane_f64(incl, 63));
-  if (wave_true(!(top <= 0.0))) {  // not every term is <= 0
+  const double p = inner ? h + (incl - a) : h;  // approximate partial sum before the block
+  double Q = -(h + readlane_f64(incl, 63));
+  if (wave_true(!neg)) {  // not every term is <= 0
     double q = 0.0;
     blk.each([&](double x) { q += fabs(x); });
-    Q = wave_sum(q) + fabs(start);
+    Q = wave_sum(q) + fabs(h);
   }
   const double delta = (4.0 * n + 256.0) * 0x1p-53 * Q;
   double s = p;
-  bool tie = false;
+  double err = 0.0;  // the additions' largest exact error; half_u where one is a tie, no more in a clean block
   const double half_u = __builtin_amdgcn_ldexp(1.0, __builtin_amdgcn_frexp_exp(p) - 54);
   blk.each([&](double x) {
     const double t = s + x;
-    tie |= fabs(x - (t - s)) == half_u;  // the addition's exact error, in a clean block
+    err = fmax(err, fabs(x - (t - s)));
     s = t;
   });
-  const bool clean = inner & (top <= 0.0) & (start <= 0.0) & !tie & (Q <= 0x1p+996) & (Q >= 0x1p-900) & (fabs(p) > delta) &
+  const bool clean = inner & neg & (h <= 0.0) & (err != half_u) & (Q <= 0x1p+996) & (Q >= 0x1p-900) & (fabs(p) > delta) &
                      (__builtin_amdgcn_frexp_exp(fabs(p) - delta) == __builtin_amdgcn_frexp_exp(fabs(s) + delta));
   const unsigned long long again = __builtin_amdgcn_ballot_w64(!clean) | 1ull;
   const double move = wave_run_scan_f64(clean ? s - p : 0.0, again);
@@ -217,18 +268,29 @@ __device__ __forceinline__ double wave_sequential_sum_of(const double *v, int n,
 // Sequential sum of v[0..n) (LDS, n wave-uniform), the same value in every
 // lane; call with the whole wave active.  v holds 64 ceil(n / 64) doubles,
 // those past n being 0.0 (adding them changes no sum).  The sum goes on from
-// `start` (a longer sum in pieces; not -0.0).  *n_events (when given) receives
-// the number of blocks added from the true sum, or -1 where the one-lane chain
-// ran.
+// `start` (a longer sum in pieces; not -0.0).  NMAX bounds n where it is known.
+// *n_events (when given) receives the number of blocks added from the true
+// sum, or -1 where the one-lane chain ran.
+//
+// A block is the 4, 8, 16 or 24 terms that 64 lanes need to cover n (n up to
+// 4,096: n / 64, from LDS).  The blocks end where v does: 4, 8 and 16 divide
+// 64 less the head, and for 24 the head is as long as that takes.
+template <int NMAX = INT_MAX>
 __device__ __forceinline__ double wave_sequential_sum(const double *v, int n, int *n_events = nullptr,
                                                       double start = 0.0) {
+  constexpr int H = kSeqSumHead;
   if (n <= 0) {
     if (n_events) *n_events = 0;
     return start;
   }
-  if (n <= 256) return wave_sequential_sum_of<4>(v, n, (n + 63) >> 6, n_events, start);
-  if (n <= 512) return wave_sequential_sum_of<8>(v, n, (n + 63) >> 6, n_events, start);
-  if (n <= kSeqSumWaveMax) return wave_sequential_sum_of<0>(v, n, (n + 63) >> 6, n_events, start);
+  if (NMAX <= H + 256 || n <= H + 256) return wave_sequential_sum_of<4>(v, H, n, n_events, start);
+  if (NMAX <= H + 512 || n <= H + 512) return wave_sequential_sum_of<8>(v, H, n, n_events, start);
+  if (NMAX <= H + 1024 || n <= H + 1024) return wave_sequential_sum_of<16>(v, H, n, n_events, start);
+  if (n <= H + 1536) {
+    const int m = ((n + 63) >> 6) % 3;  // 64 m' - head a multiple of 24
+    return wave_sequential_sum_of<24>(v, m == 0 ? 48 : m == 1 ? 40 : 32, n, n_events, start);
+  }
+  if (n <= kSeqSumWaveMax) return wave_sequential_sum_of<0>(v, H, n, n_events, start);
   if (n_events) *n_events = -1;
   double s = 0.0;
   if ((threadIdx.x & 63) == 0) s = ordered_sum(v, n, start);

@@ -365,7 +365,7 @@ void pitch_mw_kernel(PitchArgs a) {
                                   a.site_cat, a.scratch, a.cap_sites);
     return;
   }
-  MWMaster<Real, R, SPL, CAT, STRICT> m;
+  MWMaster<Real, R, MAXBD, SPL, CAT, STRICT> m;
   m.init(smem, a.model, cap);
   pitch_loop(m, taken);
 }
@@ -576,7 +576,7 @@ void optimize_mw_kernel(OptArgs a) {
                                   a.site_cat, a.scratch, a.cap_sites);
     return;
   }
-  MWMaster<Real, R, SPL, CAT, STRICT> m;
+  MWMaster<Real, R, MAXBD, SPL, CAT, STRICT> m;
   m.init(smem, a.model, cap);
   optimize_loop(m);
 }
@@ -609,7 +609,7 @@ void marginal_mw_kernel(OptArgs a) {
                                     a.site_cat, a.scratch, a.cap_sites);
     return;
   }
-  MWMaster<double, R, SPL, CAT, STRICT> m;
+  MWMaster<double, R, MAXBD, SPL, CAT, STRICT> m;
   m.init(smem, a.model, cap);
   marginal_loop(m);
 }
