@@ -15,6 +15,9 @@
 //   master: [tables, command] -> barrier A -> .............................. -> barrier B -> [sum]
 //   worker: ..................   barrier A -> [site work, wave partial sum] -> barrier B
 //
+// (Price-CAT: every wave builds a share of the tables behind barrier A, with a
+// barrier C before the site work.)
+//
 // With SPL sites per lane, worker lane j of wave w holds masked sites
 // 64*(w-1)+j + k*64*W for k < SPL.  Queries longer than the registers and LDS
 // of a workgroup hold take the streaming form (SPL = 0): a worker lane walks
@@ -59,13 +62,16 @@ struct MWShared {
   // (codes 0-3) always use rows 0-3
   int code_slot[kNucCodes];
   int slot_code[kNucCodes];
+  // Price-CAT: the proximal, distal and pendant lengths whose tables a probe
+  // builds (tflags bit 0: the first two, bit 1: the third)
+  double bl[3];
+  int tflags;
   double part[16];           // per-worker-wave sums of site logs
   long long ipart[16];       // per-worker-wave sums of site exponents
 };
 
 // LDS of one workgroup: shared header, pendant rows [n_tsl][kTable], P(prox)
-// and P(dist) [n_sl][kP], Price-CAT's exponentials [3][n_sl][4], then
-// per masked site (cap = the longest masked length the launch takes): the
+// and P(dist) [n_sl][kP], then per masked site (cap = the longest masked length the launch takes): the
 // site's log of a probe (FP64 form, rounded up to whole blocks of 64), its
 // column (the masked-site list) and in the streaming form its pendant row.
 // Gamma model: n_tsl = 1, n_sl = R (rate r uses slice r); Price-CAT: R = 1
@@ -83,12 +89,12 @@ struct MWLayout {
   static constexpr bool strict = STRICT;  // site logs summed in site order
   int n_tsl, n_sl, cap;
   bool stream;
+  MWLayout() = default;
   __host__ __device__ MWLayout(int n_tsl_, int n_sl_, int cap_, bool stream_)
       : n_tsl(n_tsl_), n_sl(n_sl_), cap(cap_), stream(stream_) {}
   __host__ __device__ size_t tbytes() const { return sizeof(Real) * (size_t)n_tsl * kTable; }
   __host__ __device__ size_t pbytes() const { return sizeof(Real) * (size_t)n_sl * kP; }
-  __host__ __device__ size_t ebytes() const { return R == 4 ? 0 : sizeof(double) * (size_t)3 * n_sl * 4; }
-  __host__ __device__ size_t off_slog() const { return head + tbytes() + 2 * pbytes() + ebytes(); }
+  __host__ __device__ size_t off_slog() const { return head + tbytes() + 2 * pbytes(); }
   __host__ __device__ size_t off_sidx() const {
     return off_slog() + (strict ? sizeof(double) * (size_t)((cap + 63) & ~63) : 0);
   }
@@ -96,9 +102,6 @@ struct MWLayout {
   __device__ Real *T(char *s) const { return reinterpret_cast<Real *>(s + head); }
   __device__ Real *Pp(char *s) const { return reinterpret_cast<Real *>(s + head + tbytes()); }
   __device__ Real *Pd(char *s) const { return reinterpret_cast<Real *>(s + head + tbytes() + pbytes()); }
-  __device__ double *E(char *s) const {
-    return reinterpret_cast<double *>(s + head + tbytes() + 2 * pbytes());
-  }
   __device__ double *slog(char *s) const { return reinterpret_cast<double *>(s + off_slog()); }
   __device__ int *sidx(char *s) const { return reinterpret_cast<int *>(s + off_sidx()); }
   __device__ int *sslot(char *s) const { return reinterpret_cast<int *>(s + off_sidx()) + cap; }
@@ -118,6 +121,89 @@ __device__ __forceinline__ void mw_copy_model(MWShared *sh, const DevModel *dm) 
   for (int t = threadIdx.x; t < 4; t += blockDim.x) { sh->l[t] = dm->l[t]; sh->statd[t] = dm->statd[t]; }
   for (int t = threadIdx.x; t < kMaxRates; t += blockDim.x) sh->rates[t] = dm->rates[t];
   for (int t = threadIdx.x; t < min(dm->n_codes, kNucCodes) * 4; t += blockDim.x) sh->lv[t] = dm->lv[t];
+}
+
+// One lane's entry of P(t) from its quad's exponentials e (lane k holds that of
+// eigenvalue k) and its rows of x and xit: the sum over k in order.
+__device__ __forceinline__ double p_entry(double e, const double (&mx)[4], const double (&mxit)[4]) {
+  double acc = 0.0;
+  acc = acc + (dpp_f64<0x00>(e) * mx[0]) * mxit[0];
+  acc = acc + (dpp_f64<0x55>(e) * mx[1]) * mxit[1];
+  acc = acc + (dpp_f64<0xAA>(e) * mx[2]) * mxit[2];
+  acc = acc + (dpp_f64<0xFF>(e) * mx[3]) * mxit[3];
+  return acc;
+}
+
+// Ambiguity codes present in the query: entry (r, i) of rows 4.. by the
+// stub's sum over the row's P entries p, which a quad's lanes hold; lane j
+// takes every fourth row.  The whole wave calls; `at` is row 0's entry, rows
+// `stride` apart.
+template <typename Real>
+__device__ __forceinline__ void ambiguity_rows(const MWShared *sh, int n_amb, double p, bool active, Real *at,
+                                               int stride) {
+  const double p0 = dpp_f64<0x00>(p), p1 = dpp_f64<0x55>(p), p2 = dpp_f64<0xAA>(p), p3 = dpp_f64<0xFF>(p);
+  if (active)
+    for (int slot = 4 + (fresh_lane() & 3); slot < 4 + n_amb; slot += 4) {
+      const double *lv = sh->lv + sh->slot_code[slot] * 4;
+      double acc = 0.0;
+      acc = acc + p0 * lv[0];
+      acc = acc + p1 * lv[1];
+      acc = acc + p2 * lv[2];
+      acc = acc + p3 * lv[3];
+      at[slot * stride] = (Real)acc;
+    }
+}
+
+// The exponentials of P(t): correctly rounded where the site logs are
+// summed in site order (the FP64 form), as the stubs' libm returns them;
+// the library's otherwise.
+template <bool STRICT>
+__device__ __forceinline__ double table_exp(double v) {
+  if constexpr (STRICT) return cr::exp(v);
+  else return exp(v);
+}
+
+// A wave's share of a Price-CAT probe's tables (sh->bl, sh->tflags): the
+// slices of categories 4 w .. 4 w + 3, then every 4 waves' further, lane
+// (category mod 4) 16 + 4 i + j taking entry (i, j) as the gamma model's does.
+// With up to 20 categories every wave of a five-wave workgroup builds at most
+// one group, in 1,900 cycles with the barrier; by the control wave alone, with
+// the others waiting, the tables took 4,280 of a probe's 10,250 cycles (2,000
+// 16S reads 14.7 -> 11.9 ms).
+template <typename Real, bool STRICT>
+__device__ __forceinline__ void cat_tables(const MWShared *sh, const MWLayout<Real, 1, STRICT> &lay, char *smem) {
+  using L = MWLayout<Real, 1, STRICT>;
+  const int lane = fresh_lane(), fl = __builtin_amdgcn_readfirstlane(sh->tflags);
+  const int n_sl = lay.n_sl, n_amb = __builtin_amdgcn_readfirstlane(sh->n_slots) - 4;
+  const int i = (lane >> 2) & 3, j = lane & 3;
+  const double m_l = sh->l[j];
+  double mx[4], mxit[4];  // the lane's row of x and of xit
+#pragma unroll
+  for (int k = 0; k < 4; k++) {
+    mx[k] = sh->x[i * 4 + k];
+    mxit[k] = sh->xit[j * 4 + k];
+  }
+  // (whole waves: quads exchange exponentials and entries)
+#pragma unroll 1
+  for (int s0 = 4 * wave_id(); s0 < n_sl; s0 += (int)blockDim.x >> 4) {
+    const int s = s0 + (lane >> 4);
+    const bool in = s < n_sl;
+    const double rate = sh->rates[in ? s : 0];
+    if (fl & 1) {
+      const double p = p_entry(table_exp<STRICT>((rate * sh->bl[0]) * m_l), mx, mxit);
+      const double d = p_entry(table_exp<STRICT>((rate * sh->bl[1]) * m_l), mx, mxit);
+      if (in) {
+        lay.Pp(smem)[s * L::kP + (lane & 15)] = (Real)p;
+        lay.Pd(smem)[s * L::kP + (lane & 15)] = (Real)d;
+      }
+    }
+    if (fl & 2) {
+      const double p = p_entry(table_exp<STRICT>((rate * sh->bl[2]) * m_l), mx, mxit);
+      Real *t = lay.T(smem) + s * L::kTable;
+      if (in) t[j * 4 + i] = (Real)p;  // one-hot row j, entry i
+      if (n_amb > 0) ambiguity_rows<Real>(sh, n_amb, (double)(Real)p, in, t + i, L::kT);
+    }
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -246,6 +332,10 @@ __device__ __forceinline__ void mw_worker(char *smem, const MWLayout<Real, R, ST
       __syncthreads();  // A
       op = sh->op;
       while (op == CMD_PROBE || op == CMD_PROBE_DIST) {
+        if constexpr (CAT) {
+          cat_tables<Real, STRICT>(sh, lay, smem);
+          __syncthreads();  // C
+        }
         Real util[SPL];
         if (op == CMD_PROBE_DIST) {
 #pragma unroll
@@ -457,6 +547,10 @@ __device__ __forceinline__ void mw_worker_stream(char *smem, const MWLayout<Real
       __syncthreads();  // A
       op = sh->op;
       while (op == CMD_PROBE || op == CMD_PROBE_DIST) {
+        if constexpr (CAT) {
+          cat_tables<Real, STRICT>(sh, lay, smem);
+          __syncthreads();  // C
+        }
         double lsum = 0.0;
         for (int i = my; i < M; i += stride) {
           const int slot = sslot[i];
@@ -547,21 +641,22 @@ struct MWMaster : ThreeTaxControl<MWMaster<Real, R, MAXBD, SPL, CAT, STRICT>> {
   static constexpr int RS = R * 4;
   MWShared *sh;
   Real *sT, *sPp, *sPd;
-  double *sE;
   const double *slog;
   int *sidx;
   int lane, n_workers, cap_sites, n_codes, n_inf, n_sl;
   int n_amb;  // ambiguity codes present in the query
   double log_R;
+  char *smem;
+  L lay;
 
   // cap: the longest masked length the launch takes (the layout's capacity)
-  __device__ __forceinline__ void init(char *smem, const DevModel *dm, int cap) {
-    const L lay = mw_layout<Real, R, STRICT>(dm, cap, SPL == 0);
+  __device__ __forceinline__ void init(char *smem_, const DevModel *dm, int cap) {
+    smem = smem_;
+    lay = mw_layout<Real, R, STRICT>(dm, cap, SPL == 0);
     sh = reinterpret_cast<MWShared *>(smem);
     sT = lay.T(smem);
     sPp = lay.Pp(smem);
     sPd = lay.Pd(smem);
-    sE = lay.E(smem);
     slog = lay.slog(smem);
     sidx = lay.sidx(smem);
     n_sl = dm->n_sl;
@@ -579,6 +674,11 @@ struct MWMaster : ThreeTaxControl<MWMaster<Real, R, MAXBD, SPL, CAT, STRICT>> {
     if (lane == 0) sh->op = op;
     __syncthreads();  // A
     if (op == CMD_EXIT) return;
+    if constexpr (CAT)
+      if (op == CMD_PROBE || op == CMD_PROBE_DIST) {
+        cat_tables<Real, STRICT>(sh, lay, smem);
+        __syncthreads();  // C
+      }
     __syncthreads();  // B
   }
 
@@ -623,33 +723,14 @@ struct MWMaster : ThreeTaxControl<MWMaster<Real, R, MAXBD, SPL, CAT, STRICT>> {
   // i*4 + j owns entry (i, j) of rate r's matrices.  It takes the exponential
   // of k = j, and a quad's four exponentials reach its lanes through DPP, so
   // nothing is staged in LDS on the probe's critical path.
-  __device__ __forceinline__ double p_entry(double e, const double (&mx)[4], const double (&mxit)[4]) const {
-    double acc = 0.0;
-    acc = acc + (dpp_f64<0x00>(e) * mx[0]) * mxit[0];
-    acc = acc + (dpp_f64<0x55>(e) * mx[1]) * mxit[1];
-    acc = acc + (dpp_f64<0xAA>(e) * mx[2]) * mxit[2];
-    acc = acc + (dpp_f64<0xFF>(e) * mx[3]) * mxit[3];
-    return acc;
-  }
-  // Ambiguity codes present in the query: entry (r, i) of rows 4.. by the
-  // stub's sum over the row's P entries p, which a quad's lanes hold; lane j
-  // takes every fourth row.  The whole wave calls; `at` is row 0's entry.
-  __device__ __forceinline__ void ambiguity_rows(double p, bool active, Real *at) const {
-    const double p0 = dpp_f64<0x00>(p), p1 = dpp_f64<0x55>(p), p2 = dpp_f64<0xAA>(p), p3 = dpp_f64<0xFF>(p);
-    if (active)
-      for (int slot = 4 + (fresh_lane() & 3); slot < 4 + n_amb; slot += 4) {
-        const double *lv = sh->lv + sh->slot_code[slot] * 4;
-        double acc = 0.0;
-        acc = acc + p0 * lv[0];
-        acc = acc + p1 * lv[1];
-        acc = acc + p2 * lv[2];
-        acc = acc + p3 * lv[3];
-        at[slot * L::kT] = (Real)acc;
-      }
-  }
   __device__ __forceinline__ void tables(bool new_pend, bool new_dist) {
-    if constexpr (CAT) {
-      cat_tables(new_pend, new_dist);
+    if constexpr (CAT) {  // built by all waves once the command is out
+      if (fresh_lane() == 0) {
+        sh->bl[0] = prox_bl;
+        sh->bl[1] = dist_bl;
+        sh->bl[2] = pend_bl;
+        sh->tflags = (new_dist ? 1 : 0) | (new_pend ? 2 : 0);
+      }
       return;
     }
     const int lane = fresh_lane();
@@ -661,78 +742,20 @@ struct MWMaster : ThreeTaxControl<MWMaster<Real, R, MAXBD, SPL, CAT, STRICT>> {
       mxit[k] = sh->xit[(lane & 3) * 4 + k];
     }
     if (new_dist) {
-      const double p = p_entry(texp((m_rate * prox_bl) * m_l), mx, mxit);
-      const double d = p_entry(texp((m_rate * dist_bl) * m_l), mx, mxit);
+      const double p = p_entry(table_exp<STRICT>((m_rate * prox_bl) * m_l), mx, mxit);
+      const double d = p_entry(table_exp<STRICT>((m_rate * dist_bl) * m_l), mx, mxit);
       if (lane < R * 16) {
         sPp[(lane >> 4) * L::kP + (lane & 15)] = (Real)p;
         sPd[(lane >> 4) * L::kP + (lane & 15)] = (Real)d;
       }
     }
     if (new_pend) {
-      const double p = p_entry(texp((m_rate * pend_bl) * m_l), mx, mxit);
+      const double p = p_entry(table_exp<STRICT>((m_rate * pend_bl) * m_l), mx, mxit);
       const int j = lane & 3, ri = (lane >> 2) & (R * 4 - 1);
       // One-hot characters: their evolved rows are columns of P (every other
       // product in gemmish_c is an exact zero), row j entry (r, i) = P[r][i][j].
       if (lane < R * 16) sT[j * L::kT + ri] = (Real)p;
-      if (n_amb > 0) ambiguity_rows(p, lane < R * 16, sT + ri);
-    }
-  }
-
-  // The exponentials of P(t): correctly rounded where the site logs are
-  // summed in site order (the FP64 form), as the stubs' libm returns them;
-  // the library's otherwise.
-  static __device__ __forceinline__ double texp(double v) {
-    if constexpr (STRICT) return cr::exp(v);
-    else return exp(v);
-  }
-
-  // Price-CAT tables: the same sums for every category slice.  The
-  // exponentials (category s, eigenvalue k at 4 s + k) go through LDS, a lane
-  // one of 64 at a time, so each is taken once; then lane (s mod 4) 16 + i 4 +
-  // j forms entry (i, j) of every fourth category's matrices, with its rows of
-  // x and xit in registers, and the ambiguity rows from its quad.
-  __device__ __forceinline__ void cat_exps(double bl, double *e) {
-    const int lane = fresh_lane();
-    const double m_l = sh->l[lane & 3];
-    for (int t = lane; t < 4 * n_sl; t += 64) e[t] = texp((sh->rates[t >> 2] * bl) * m_l);
-  }
-  static __device__ __forceinline__ double cat_entry(const double *e, const double (&mx)[4], const double (&mxit)[4]) {
-    double acc = 0.0;
-#pragma unroll
-    for (int k = 0; k < 4; k++) acc = acc + (e[k] * mx[k]) * mxit[k];
-    return acc;
-  }
-  __device__ __forceinline__ void cat_tables(bool new_pend, bool new_dist) {
-    double *e0 = sE, *e1 = sE + 4 * n_sl, *e2 = sE + 8 * n_sl;  // proximal, distal, pendant
-    if (new_dist) {
-      cat_exps(prox_bl, e0);
-      cat_exps(dist_bl, e1);
-    }
-    if (new_pend) cat_exps(pend_bl, e2);
-    wave_lds_sync();
-    const int lane = fresh_lane();
-    double mx[4], mxit[4];
-#pragma unroll
-    for (int k = 0; k < 4; k++) {
-      mx[k] = sh->x[(lane & 12) + k];
-      mxit[k] = sh->xit[(lane & 3) * 4 + k];
-    }
-    const int i = (lane >> 2) & 3, j = lane & 3;
-    if (new_dist) {
-#pragma unroll 2
-      for (int s = lane >> 4; s < n_sl; s += 4) {
-        sPp[s * L::kP + (lane & 15)] = (Real)cat_entry(e0 + 4 * s, mx, mxit);
-        sPd[s * L::kP + (lane & 15)] = (Real)cat_entry(e1 + 4 * s, mx, mxit);
-      }
-    }
-    if (new_pend) {
-#pragma unroll 2
-      for (int s0 = 0; s0 < n_sl; s0 += 4) {  // whole waves: quads exchange entries
-        const int s = s0 + (lane >> 4);
-        const double p = cat_entry(e2 + 4 * (s < n_sl ? s : 0), mx, mxit);
-        if (s < n_sl) sT[s * L::kTable + j * 4 + i] = (Real)p;  // one-hot row j, entry i
-        if (n_amb > 0) ambiguity_rows((double)(Real)p, s < n_sl, sT + s * L::kTable + i);
-      }
+      if (n_amb > 0) ambiguity_rows<Real>(sh, n_amb, p, lane < R * 16, sT + ri, L::kT);
     }
   }
 
