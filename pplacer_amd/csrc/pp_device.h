@@ -1,13 +1,6 @@
 // Device-side building blocks shared by the placement kernels: wavefront and
-// block reductions, the stage-1 ranking key, and the three-taxon engine that
-// runs Three_tax.optimize (three_tax.ml:70-83) with the GSL Brent minimiser
-// restated on the GPU.
-//
-// Execution model of the engine: one workgroup owns one (query, edge) at a
-// time; lane j holds masked site j of the query (pend GLV code, distal and
-// proximal GLV rows, the cached (pi*prox_ev)*dist_ev products).  Every lane
-// runs the same scalar Brent / baseball logic on block-uniform values, so the
-// control flow is uniform and each likelihood probe is one collective call.
+// block reductions, values kept in scalar registers, the stage-1 ranking key
+// and the states of Three_tax.optimize (three_tax.ml:70-83).
 #pragma once
 
 #include <hip/hip_runtime.h>
