@@ -432,9 +432,7 @@ struct ProtMaster : ThreeTaxControl<ProtMaster<Real, R>> {
       sh->tile_next = 0;
     }
     command(new_dist ? CMD_PROBE_DIST : CMD_PROBE);
-    const double pv = sh->part[fresh_lane() & 15];  // lane w: worker wave w's partial, added in wave order
-    double tot = readlane_f64(pv, 0);
-    for (int w = 1; w < n_workers; w++) tot += readlane_f64(pv, w);
+    const double tot = sum_parts<7>(sh->part);  // in wave order
     c_pend = scalar(pend_bl);
     c_dist = scalar(dist_bl);
     c_prox = scalar(prox_bl);
