@@ -329,7 +329,8 @@ def main():
                     "phase_frac": st_main["pitch_u2_tflops"] / peak if st_main["pitch_u2_tflops"] else None,
                     "work": "reference U2 flops of the pitched probes: (2RS^2+4RS) per masked site "
                             "of a pendant probe, (4RS^2+4RS) of a distal probe"}
-        if S == 4 and real == "double" and not args.tune:
+        # (shorter chunks spread the phase over streams)
+        if S == 4 and real == "double" and not args.tune and args.queries > 32768 * -(-args.queries // 65536):
             roofline["launch_note"] = ("the FP64 baseball launches run one after another on the main "
                                        "stream (launch shape pitch_streams[0] = 0), so each launch's "
                                        "duration is its own; --tune may spread them over streams "

@@ -333,10 +333,13 @@ int pp_synchronize(pp_ctx *ctx);
  *   pitch_streams[f], refine_streams[f]: streams over which the 4-state
  *     baseball phase and the refinement phase spread their masked-length
  *     buckets, for form f (0 = PP_FP64, 1 = PP_FP32); 0 runs them one after
- *     another on the main stream; at most PP_MAX_BUCKET_STREAMS.  Until a
- *     shape is set, passes in chunks of at most 32,768 queries spread the
- *     baseball and -p phases over at least 4 streams; after that the -p phase
- *     runs on the main stream, as 20-state passes always do.
+ *     another on the main stream; at most PP_MAX_BUCKET_STREAMS.  While both
+ *     counts of a form are the defaults (0 and 4 for PP_FP64, 8 and 4 for
+ *     PP_FP32), its passes in chunks of at most 32,768 queries run as a short
+ *     pass: the baseball and -p phases spread over at least 4 streams, and
+ *     small neighbouring buckets share a launch.  Any other pair is taken as
+ *     it stands, with the -p phase on the main stream.  20-state passes
+ *     always run on the main stream.
  *   chunk: queries per device chunk (stage 1 of the next chunk overlaps
  *     stage 2 of the current one), 1 .. PP_MAX_CHUNK, further capped so that a
  *     chunk's scores ([chunk][n_edges] doubles) stay under 2 GiB.

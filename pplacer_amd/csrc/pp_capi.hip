@@ -55,7 +55,7 @@ static_assert(kChunk <= PP_MAX_CHUNK, "default chunk out of range");
 // 2,000 taxa.
 constexpr int kPitchStreams[2] = {0, 8};
 constexpr int kRefineStreams[2] = {4, 4};
-// Until a launch shape is given (pp_launch_config_set), 4-state passes of
+// While a form's two stream counts are these defaults, its 4-state passes of
 // chunks of at most kForkQueries run their baseball and -p phases over at least
 // kForkStreams streams: a bucket's launch is then a few rounds of the work
 // queue at most, and ends on a tail of a few long queries that the other
@@ -108,7 +108,6 @@ struct pp_ctx {
   hipStream_t s1 = nullptr;           // stage 1 of the next chunk
   hipStream_t bs[kBucketStreams] = {};  // concurrent stage-2 buckets
   hipStream_t cur = nullptr;          // the stream the launch helpers use
-  bool launch_given = false;          // pp_launch_config_set has been called
   pp_launch_config launch{{kPitchStreams[0], kPitchStreams[1]}, {kRefineStreams[0], kRefineStreams[1]}, kChunk, 0};
   // graph mode: captured chunk loops by plan key (most recent last; a pass
   // and the FP64 re-placement of its FP32 failures keep one each)
@@ -1114,7 +1113,15 @@ void merge_buckets(const pp_ctx *c, std::vector<std::vector<int>> &buckets, bool
   }
 }
 
-int place_pass(pp_ctx *c, const pp_prefs *prefs, int precision, pp_stats *stats) {
+// Whether form f's streams are the default shape's, under which short chunks
+// take the plan of kForkQueries and merge_buckets.  A property of the shape in
+// force alone: setting what pp_launch_config_get reports changes nothing.
+bool default_streams(const pp_launch_config &l, int f) {
+  return l.pitch_streams[f] == kPitchStreams[f] && l.refine_streams[f] == kRefineStreams[f];
+}
+
+// form: whose streams of the launch shape the pass takes (0 or 1)
+int place_pass(pp_ctx *c, const pp_prefs *prefs, int precision, int form, pp_stats *stats) {
   CHECK(prefs, PP_EINVAL, "prefs is null");
   CHECK(precision == PP_FP64 || precision == PP_FP32, PP_EINVAL, "precision must be PP_FP64 or PP_FP32");
   CHECK(prefs->keep_at_most >= 0 && prefs->keep_at_most <= 64, PP_EINVAL, "keep_at_most must be in 0..64");
@@ -1176,12 +1183,12 @@ int place_pass(pp_ctx *c, const pp_prefs *prefs, int precision, pp_stats *stats)
   // launch's duration is the kernel's own (4 streams measured within 1% at
   // 50,000-query chunks), and a tuner may set them.  The 20-state kernels
   // share one scratch buffer and do not fork.
-  const bool fork = c->model.S == 4 && !c->launch_given && Q <= (int64_t)kForkQueries * n_chunks;
+  const bool fork = c->model.S == 4 && default_streams(c->launch, form) && Q <= (int64_t)kForkQueries * n_chunks;
   const int pitch_streams = c->model.S != 4 ? 0
-                            : fork ? std::max(c->launch.pitch_streams[s2_fp32], kForkStreams)
-                                   : c->launch.pitch_streams[s2_fp32];
+                            : fork ? std::max(c->launch.pitch_streams[form], kForkStreams)
+                                   : c->launch.pitch_streams[form];
   const int marg_streams = fork ? kForkStreams : 0;
-  const int refine_streams = c->model.S == 4 ? c->launch.refine_streams[s2_fp32 ? 1 : 0] : 0;
+  const int refine_streams = c->model.S == 4 ? c->launch.refine_streams[form] : 0;
   hipEvent_t e_t0 = pool.get(), e_t1 = pool.get();
   CHECK(e_t0 && e_t1, PP_EDEVICE, "hipEventCreate failed");
   HIPCHECK(hipEventRecord(e_t0, c->stream));
@@ -1291,7 +1298,7 @@ int place_pass(pp_ctx *c, const pp_prefs *prefs, int precision, pp_stats *stats)
   uint64_t key = 0;
   if (graph) {
     PlanKey h;
-    h.add(Q); h.add(K); h.add(precision); h.add(*prefs); h.add(c->launch); h.add(n_chunks);
+    h.add(Q); h.add(K); h.add(precision); h.add(form); h.add(*prefs); h.add(c->launch); h.add(n_chunks);
     h.add_vec(cq0); h.add_vec(t_off);
     for (const auto &bo : boffs) h.add_vec(bo);
     const void *ptrs[] = {d_out, d_nout, d_status, d_scores, d_res, d_nres, d_kept, d_nkeep, d_qlist,
@@ -1621,12 +1628,8 @@ int replace_in_fp64(pp_ctx *c, const pp_prefs *prefs, const std::vector<int> &id
   c->qstat.assign(n, PP_Q_OK);
   // A handful of queries spread over the stage-2 classes: their launches run
   // concurrently on the FP32 form's streams rather than one after another.
-  const pp_launch_config launch = c->launch;
-  c->launch.pitch_streams[0] = launch.pitch_streams[1];
-  c->launch.refine_streams[0] = launch.refine_streams[1];
   pp_stats sub{};
-  int st = place_pass(c, prefs, PP_FP64, &sub);
-  c->launch = launch;
+  int st = place_pass(c, prefs, PP_FP64, 1, &sub);
   swap_bufs();
   c->Q = Q;
   c->order = std::move(order_s);
@@ -1654,7 +1657,7 @@ int replace_in_fp64(pp_ctx *c, const pp_prefs *prefs, const std::vector<int> &id
 // A placement pass over the resident queries; in the 4-state FP32 form the
 // queries failing the prox_bl assertion are then placed again in FP64.
 int place_resident(pp_ctx *c, const pp_prefs *prefs, int precision, pp_stats *stats) {
-  int st = place_pass(c, prefs, precision, stats);
+  int st = place_pass(c, prefs, precision, precision == PP_FP32, stats);
   if (st || precision != PP_FP32 || !stage2_fp32_ok(c) || c->Q == 0) return st;
   std::vector<int> hs(c->Q), idx;
   HIPCHECK(hipMemcpy(hs.data(), c->b_status.p, (size_t)c->Q * 4, hipMemcpyDeviceToHost));
@@ -1945,7 +1948,6 @@ int pp_launch_config_set(pp_ctx *c, const pp_launch_config *cfg) {
   CHECK(cfg->chunk >= 1 && cfg->chunk <= PP_MAX_CHUNK, PP_EINVAL, "chunk must be in 1..PP_MAX_CHUNK");
   CHECK(cfg->graph == 0 || cfg->graph == 1, PP_EINVAL, "graph must be 0 or 1");
   c->launch = *cfg;
-  c->launch_given = true;
   return PP_OK;
 }
 

@@ -317,8 +317,8 @@ class Placer:
     def launch_config(self) -> dict:
         """The pass's launch shape: streams per stage-2 phase and form
         (index 0 = FP64, 1 = FP32), queries per device chunk, and whether the
-        pass's launches are captured into a replayed HIP graph.  Until a shape
-        is set, passes in short chunks use more streams than this says
+        pass's launches are captured into a replayed HIP graph.  With a form's
+        default streams, passes in short chunks spread further than this says
         (include/pplacer_hip.h, pp_launch_config)."""
         cfg = LaunchConfig()
         check(lib().pp_launch_config_get(self._ctx, C.byref(cfg)), "launch_config_get")
