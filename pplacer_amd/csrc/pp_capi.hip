@@ -1299,6 +1299,14 @@ int place_pass(pp_ctx *c, const pp_prefs *prefs, int precision, int form, pp_sta
   if (graph) {
     PlanKey h;
     h.add(Q); h.add(K); h.add(precision); h.add(form); h.add(*prefs); h.add(c->launch); h.add(n_chunks);
+    // the model, tree and longest masked length the kernels and their
+    // arguments are chosen by, and the prior's kind (buffers keep their
+    // addresses when these change)
+    int max_m = 0;
+    for (int q = 0; q < Q; q++)
+      if (c->qstat[q] == PP_Q_OK) max_m = std::max(max_m, c->qM[q]);
+    h.add(c->model.S); h.add(c->model.R); h.add(c->model.n_cats); h.add(N); h.add(E); h.add(max_m);
+    h.add(marg_proto.prior_kind);
     h.add_vec(cq0); h.add_vec(t_off);
     for (const auto &bo : boffs) h.add_vec(bo);
     const void *ptrs[] = {d_out, d_nout, d_status, d_scores, d_res, d_nres, d_kept, d_nkeep, d_qlist,

@@ -1,7 +1,9 @@
 """The plan of a short pass (include/pplacer_hip.h, pp_launch_config) belongs to
 the launch shape in force: it holds whenever a form's stream counts are the
 defaults, however they came to be set, and ends where they are not.  The number
-of baseball launches shows which plan a pass took."""
+of baseball launches shows which plan a pass took.  A captured pass is replayed
+only for the plan, model, tree and prior it was captured with."""
+import numpy as np
 import pytest
 
 pytestmark = pytest.mark.gpu
@@ -79,3 +81,77 @@ def test_tuner_times_the_plan_in_force_first(reads, monkeypatch):
     # the untimed first pass and the first trial: the same shape, the same launches
     assert seen[0] == seen[1] and seen[0][0] == default == trials[0][0]
     assert seen[2][1] > seen[1][1]  # two streams asked for: a launch per class
+
+
+def _graph_equals_eager(pl, queries, prefs, what):
+    """A graph pass (captured or replayed), an eager one and a replay."""
+    from pplacer_amd import placer
+    got = []
+    for graph in (1, 0, 1):
+        _print_case("graph %d, %s" % (graph, what))
+        pl.set_launch_config(graph=graph)
+        rows, status, _ = pl.place(queries, prefs=prefs, precision=placer.PP_FP64)
+        got.append((rows, list(status)))
+    assert got[0] == got[1] and got[2] == got[1], what
+    return got[1]
+
+
+def test_graph_follows_the_prior(reads):
+    """The prior's kind is an argument of a captured -p launch."""
+    from pplacer_amd import placer
+    pl, queries = reads
+    prefs = placer.default_prefs(calc_pp=True)
+    try:
+        flat = _graph_equals_eager(pl, queries, prefs, "flat prior")
+        pl.set_prior("uniform")
+        uniform = _graph_equals_eager(pl, queries, prefs, "uniform prior")
+        assert uniform != flat
+        pl.set_prior("flat")
+        assert _graph_equals_eager(pl, queries, prefs, "flat prior again") == flat
+    finally:
+        pl.set_prior("flat")
+        pl.set_launch_config(graph=0)
+
+
+def test_graph_follows_model_and_tree():
+    """One context whose model and tree change between passes of the same
+    queries: buffers keep their addresses, a captured pass must not be kept."""
+    from pplacer_amd import placer, synth
+    wl = synth.make_workload("gtr12", seed=5)
+    small = synth.make_workload("gtr12", seed=6, n_taxa=9)
+    pl, queries, statd, rates = placer.setup_from_workload(wl, premasked=False)
+    prefs = placer.default_prefs()
+    n = len(queries[0])
+    try:
+        four = _graph_equals_eager(pl, queries, prefs, "four rates")
+        pl.build_model(wl.exch, statd, [1.0])
+        pl.set_tree(wl.tree, wl.leaf_seqs(), n)
+        one = _graph_equals_eager(pl, queries, prefs, "one rate")
+        pl.build_model_cat(wl.exch, statd, [0.3, 1.0, 2.0], np.arange(n) % 3)
+        pl.set_tree(wl.tree, wl.leaf_seqs(), n)
+        cat = _graph_equals_eager(pl, queries, prefs, "three categories")
+        pl.build_model(wl.exch, statd, rates)
+        pl.set_tree(small.tree, small.leaf_seqs(), n)
+        other = _graph_equals_eager(pl, queries, prefs, "another tree")
+        pl.set_tree(wl.tree, wl.leaf_seqs(), n)
+        assert _graph_equals_eager(pl, queries, prefs, "four rates again") == four
+        assert len({str(r) for r in (four, one, cat, other)}) == 4
+    finally:
+        pl.close()
+
+
+def test_graph_follows_the_longest_protein():
+    """20 states: one class, whose capacity is the longest masked length."""
+    from pplacer_amd import placer, synth
+    wl = synth.make_workload("prot10", seed=4, n_queries=1, n_columns=300)
+    pl, _, _, _ = placer.setup_from_workload(wl, premasked=False)
+    prefs = placer.default_prefs()
+    rows = list(wl.leaf_seqs().values())
+    n = len(rows[0])
+    try:
+        pl.place(rows, prefs=prefs)  # the buffers' largest sizes from the start
+        for m in (20, n, 20):
+            got = _graph_equals_eager(pl, [r[:m] + "-" * (n - m) for r in rows], prefs, "proteins of %d sites" % m)
+            assert all(s == 0 for s in got[1])
+    finally:
+        pl.close()
