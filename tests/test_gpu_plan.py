@@ -155,3 +155,42 @@ def test_graph_follows_the_longest_protein():
             assert all(s == 0 for s in got[1])
     finally:
         pl.close()
+
+
+# around the classes' ends, the two-sites-a-lane classes, and (for four rates
+# past 960 sites, else past 1,920) the streaming class
+PLAN_LENGTHS = [30, 64, 65, 200, 300, 449, 700, 960, 961, 1200, 1500, 1569, 1900, 1920, 1921, 2100, 2200]
+
+
+@pytest.mark.parametrize("form", ["fp64", "fp32"])
+@pytest.mark.parametrize("model", ["four_rates", "one_rate", "cat20"])
+def test_short_pass_plan_equals_main_stream(model, form):
+    """All classes at once, the streaming one beside the others, in one chunk and
+    in several: the results are the main stream's, bit for bit, with -p."""
+    from pplacer_amd import placer
+    from tests.test_gpu_streaming import long_workload, masked, rows_of
+    wl = long_workload(22)
+    wl.n_cats = 4 if model == "four_rates" else 1
+    prec = placer.PP_FP64 if form == "fp64" else placer.PP_FP32
+    prefs = placer.default_prefs(calc_pp=True, max_pitches=6, keep_at_most=3)
+    pl, _, statd, _ = placer.setup_from_workload(wl)
+    if model == "cat20":
+        rng = np.random.default_rng(20)
+        pl.build_model_cat(wl.exch, statd, np.sort(rng.uniform(0.05, 3.0, 20)), rng.integers(0, 20, 2200))
+        pl.set_tree(wl.tree, wl.leaf_seqs(), 2200)
+    try:
+        rows = rows_of(wl)
+        queries = [masked(rows[(i + 5 * k) % len(rows)], m) for k in range(3) for i, m in enumerate(PLAN_LENGTHS)]
+        default = pl.launch_config()
+        got = {}
+        for name, shape in (("one chunk", default), ("four chunks", dict(default, chunk=13)),
+                            ("main stream", dict(default, **SERIAL))):
+            _print_case("gtr12 seed 22, 2,200 columns, %s, %s, %s" % (model, form, name))
+            pl.set_launch_config(**shape)
+            rows_, status, _ = pl.place(queries, prefs=prefs, precision=prec)
+            got[name] = rows_, list(status)
+    finally:
+        pl.close()
+    assert all(s == 0 for s in got["main stream"][1])
+    assert got["one chunk"] == got["main stream"]
+    assert got["four chunks"] == got["main stream"]
