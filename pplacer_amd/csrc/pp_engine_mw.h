@@ -52,8 +52,6 @@ namespace pp {
 // CMD_PROBE_DIST: a probe whose proximal/distal lengths changed (re-evolve)
 enum { CMD_EXIT = 0, CMD_QUERY = 1, CMD_GATHER = 2, CMD_PROBE = 3, CMD_PROBE_DIST = 4 };
 
-constexpr int kNucCodes = 16;  // character codes of the 4-state models
-
 struct MWShared {
   double x[16], l[4], xit[16], statd[4], rates[kMaxRates];
   double lv[kNucCodes * 4];
@@ -121,7 +119,7 @@ __device__ __forceinline__ void mw_copy_model(MWShared *sh, const DevModel *dm) 
   for (int t = threadIdx.x; t < 4; t += blockDim.x) { sh->l[t] = dm->l[t]; sh->statd[t] = dm->statd[t]; }
   for (int t = threadIdx.x; t < kMaxRates; t += blockDim.x) sh->rates[t] = dm->rates[t];
   for (int t = threadIdx.x; t < 16; t += blockDim.x) sh->part[t] = 0.0;
-  for (int t = threadIdx.x; t < min(dm->n_codes, kNucCodes) * 4; t += blockDim.x) sh->lv[t] = dm->lv[t];
+  for (int t = threadIdx.x; t < kNucCodes * 4; t += blockDim.x) sh->lv[t] = dm->lv[t];
 }
 
 // One lane's entry of P(t) from its quad's exponentials e (lane k holds that of

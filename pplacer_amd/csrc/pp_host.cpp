@@ -215,6 +215,8 @@ static void fill_codes(HostModel &m) {
     static const struct { const char *c; int bits; } tab[] = {
         {"A", 1}, {"C", 2}, {"G", 4}, {"T", 8}, {"R", 5}, {"Y", 10}, {"M", 3}, {"K", 12},
         {"S", 6}, {"W", 9}, {"H", 11}, {"B", 14}, {"V", 7}, {"D", 13}, {"NX", 15}};
+    // the stage-2 kernels' tables hold one row a code ("-?" is the last)
+    static_assert(sizeof(tab) / sizeof(tab[0]) + 1 == kNucCodes, "4-state character codes");
     for (auto &t : tab) {
       double v[4];
       for (int i = 0; i < 4; i++) v[i] = (t.bits >> i) & 1 ? 1. : 0.;
@@ -225,6 +227,7 @@ static void fill_codes(HostModel &m) {
     add("-?", ones);
   } else {
     static const char code[] = "ARNDCQEGHILKMFPSTWYV";
+    static_assert(20 + 5 <= kMaxCodes, "20-state character codes (B, J, Z, X and -? besides the 20)");
     for (int i = 0; i < 20; i++) {
       double v[20] = {0};
       v[i] = 1.;

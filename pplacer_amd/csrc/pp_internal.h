@@ -12,7 +12,8 @@ namespace pp {
 
 constexpr int kMaxStates = 20;
 constexpr int kMaxRates = 32;  // gamma rates, or Price-CAT categories
-constexpr int kMaxCodes = 32;
+constexpr int kMaxCodes = 32;  // character codes of any model
+constexpr int kNucCodes = 16;  // character codes of the 4-state models
 
 // Model as the kernels see it.  Character codes: index into lv[]; codes
 // >= n_inf are the non-informative '-' and '?' (alignment.ml:235).
