@@ -67,7 +67,6 @@ constexpr int kRefineStreams[2] = {4, 4};
 // -> 149.  Larger chunks gain 2% at most and stay on the main stream, where a
 // launch's duration is the kernel's own.
 constexpr int kForkQueries = 32768, kForkStreams = 4;
-constexpr int kProtBlock = 512;   // lanes of a 20-state stage-2 workgroup (master + workers)
 
 struct DBuf {
   void *p = nullptr;

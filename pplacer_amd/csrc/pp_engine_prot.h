@@ -34,6 +34,8 @@
 namespace pp {
 
 constexpr int kProtS = 20;
+constexpr int kProtBlock = 512;                     // lanes of a workgroup (master + workers)
+constexpr int kProtWorkers = kProtBlock / 64 - 1;   // worker waves
 
 struct ProtShared {
   double x[kProtS * kProtS], xit[kProtS * kProtS];  // [i][k], [j][k]
@@ -46,8 +48,8 @@ struct ProtShared {
   // distal, bit 1: pendant), and the number of character codes
   int tflags, n_codes;
   int tile_next;  // FP32 form: the next 64-pair tile a worker wave takes
-  double part[16];      // per-worker-wave sums of site logs
-  long long ipart[16];  // per-worker-wave sums of site exponents
+  double part[kProtWorkers];      // per-worker-wave sums of site logs
+  long long ipart[kProtWorkers];  // per-worker-wave sums of site exponents
 };
 
 struct ProtLayout {
@@ -354,7 +356,7 @@ struct ProtMaster : ThreeTaxControl<ProtMaster<Real, R>> {
   static constexpr bool kF32 = std::is_same<Real, float>::value;
   ProtShared *sh;
   int *sidx;
-  int lane, n_workers, cap_sites, n_inf, n_sl;
+  int lane, cap_sites, n_inf, n_sl;
   double log_R;
 
   __device__ __forceinline__ void init(char *smem, const DevModel *dm, int cap_pairs) {
@@ -362,7 +364,6 @@ struct ProtMaster : ThreeTaxControl<ProtMaster<Real, R>> {
     sh = reinterpret_cast<ProtShared *>(smem);
     sidx = ProtLayout::sidx(smem);
     lane = threadIdx.x & 63;
-    n_workers = (blockDim.x >> 6) - 1;
     cap_sites = cap_pairs / R;
     n_inf = dm->n_inf;
     log_R = dm->log_R;
@@ -397,7 +398,7 @@ struct ProtMaster : ThreeTaxControl<ProtMaster<Real, R>> {
   __device__ __forceinline__ void gather(int loc) {
     if (lane == 0) sh->loc = loc;
     command(CMD_GATHER);
-    const long long es = wave_sum_ll(lane < n_workers ? sh->ipart[lane] : 0);
+    const long long es = wave_sum_ll(lane < kProtWorkers ? sh->ipart[lane] : 0);
     esum = scalar((double)es);
     c_dist = c_prox = __builtin_nan("");
     have_last = false;
@@ -432,7 +433,7 @@ struct ProtMaster : ThreeTaxControl<ProtMaster<Real, R>> {
       sh->tile_next = 0;
     }
     command(new_dist ? CMD_PROBE_DIST : CMD_PROBE);
-    const double tot = sum_parts<7>(sh->part);  // in wave order
+    const double tot = sum_parts<kProtWorkers>(sh->part);  // in wave order
     c_pend = scalar(pend_bl);
     c_dist = scalar(dist_bl);
     c_prox = scalar(prox_bl);

@@ -412,7 +412,7 @@ struct ProtOcc {
 };
 
 template <typename Real, int R>
-__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(ProtOcc<Real>::waves)))
+__global__ __launch_bounds__(kProtBlock) __attribute__((amdgpu_waves_per_eu(ProtOcc<Real>::waves)))
 void pitch_prot_kernel(PitchArgs a) {
   extern __shared__ __align__(16) char smem[];
   const size_t end = prot_setup<Real, R>(smem, a.model, a.N);
@@ -582,7 +582,7 @@ void optimize_mw_kernel(OptArgs a) {
 }
 
 template <typename Real, int R>
-__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(ProtOcc<Real>::waves)))
+__global__ __launch_bounds__(kProtBlock) __attribute__((amdgpu_waves_per_eu(ProtOcc<Real>::waves)))
 void optimize_prot_kernel(OptArgs a) {
   extern __shared__ __align__(16) char smem[];
   (void)prot_setup<Real, R>(smem, a.model, a.N);
@@ -615,7 +615,7 @@ void marginal_mw_kernel(OptArgs a) {
 }
 
 template <int R>
-__global__ __launch_bounds__(512) void marginal_prot_kernel(OptArgs a) {
+__global__ __launch_bounds__(kProtBlock) void marginal_prot_kernel(OptArgs a) {
   extern __shared__ __align__(16) char smem[];
   prot_copy_model(reinterpret_cast<ProtShared *>(smem), a.model);
   __syncthreads();
