@@ -613,16 +613,19 @@ size_t stage2_lds(const pp_ctx *c, int bd, size_t taken, int spl, int stream_cap
 }
 // LDS by which a masked length is classed and accepted: a fixed account of the
 // FP64 workgroup (header and tables, 16 bytes of log sum and 4 or 8 of list a
-// site, 1 KB, the pitch kernel's flags, products), never less than the layout
-// takes, so that neither the class limits nor the longest query the GPU path
-// takes move when the layout does.
+// site, 1 KB, the pitch kernel's flags, products), so that neither the class
+// limits nor the longest query the GPU path takes move when the layout does;
+// a layout that has come to take more counts by itself, so that no query is
+// accepted whose launch would fail.
 size_t accept_lds(const pp_ctx *c, int bd, size_t taken, int spl, int stream_cap) {
   const size_t cap = spl == 0 ? stream_cap : (bd - 64) * spl, R = c->model.R, n_sl = c->model.n_sl();
   const size_t n_tsl = c->model.n_cats > 0 ? c->model.n_cats : 1;
   const auto align = [](size_t v) { return (v + 15) & ~size_t(15); };
   const size_t base = 2144 + 8 * n_tsl * 32 * R * 4 + 2 * 8 * n_sl * 16 + 8 * 3 * n_sl * 4 + 16 * cap + 1024;
   const size_t products = R == 4 ? MWProducts<double, 16>::bytes((int)cap) : MWProducts<double, 4>::bytes((int)cap);
-  return align(align(base + 4 * cap * (spl ? 1 : 2)) + taken) + (spl ? products : 0);
+  const size_t account = align(align(base + 4 * cap * (spl ? 1 : 2)) + taken) + (spl ? products : 0);
+  return std::max(account, R == 4 ? stage2_lds<double, 4, true>(c, bd, taken, spl, stream_cap)
+                                  : stage2_lds<double, 1, true>(c, bd, taken, spl, stream_cap));
 }
 
 // Whether the FP32 form runs stage 2 in FP32.  The 20-state engine evaluates
