@@ -199,7 +199,6 @@ template <int CAP>
 __device__ __forceinline__ double wave_sequential_sum_of(const double *v, int head, int n, int *n_events,
                                                          double start) {
   SeqSumBlock<CAP> blk;
-  blk.load(v + head, n - head);
   // The head's loads eight ahead, its additions among those of the blocks and the
   // scan's steps, as written (left to itself the compiler finished the scan
   // first and then waited for LDS at every eighth addition)
