@@ -199,13 +199,14 @@ template <int CAP>
 __device__ __forceinline__ double wave_sequential_sum_of(const double *v, int head, int n, int *n_events,
                                                          double start) {
   SeqSumBlock<CAP> blk;
-  // The head's loads eight ahead, its additions among those of the blocks and the
+  blk.load(v + head, n - head);
+  // The block's loads first (after the head's they cost 400 reads with -p 1.7%),
+  // the head's eight ahead, its additions among those of the blocks and the
   // scan's steps, as written (left to itself the compiler finished the scan
   // first and then waited for LDS at every eighth addition)
   double h = start, y[8];
 #pragma unroll
   for (int j = 0; j < 8; j++) y[j] = v[j];
-  blk.load(v + head, n - head);
   double a = 0.0;
   double top = 0.0;
   blk.each([&](double x) {
