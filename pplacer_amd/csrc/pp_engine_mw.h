@@ -119,7 +119,7 @@ __device__ __forceinline__ void mw_copy_model(MWShared *sh, const DevModel *dm) 
   for (int t = threadIdx.x; t < 4; t += blockDim.x) { sh->l[t] = dm->l[t]; sh->statd[t] = dm->statd[t]; }
   for (int t = threadIdx.x; t < kMaxRates; t += blockDim.x) sh->rates[t] = dm->rates[t];
   for (int t = threadIdx.x; t < 16; t += blockDim.x) sh->part[t] = 0.0;
-  for (int t = threadIdx.x; t < kNucCodes * 4; t += blockDim.x) sh->lv[t] = dm->lv[t];
+  for (int t = threadIdx.x; t < min(dm->n_codes, kNucCodes) * 4; t += blockDim.x) sh->lv[t] = dm->lv[t];
 }
 
 // One lane's entry of P(t) from its quad's exponentials e (lane k holds that of
