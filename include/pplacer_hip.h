@@ -345,8 +345,9 @@ int pp_synchronize(pp_ctx *ctx);
  *     chunk's scores ([chunk][n_edges] doubles) stay under 2 GiB.
  *   graph: 1 captures the pass's stage-1 and stage-2 launches (every chunk,
  *     every stream) into a HIP graph and replays it on the next passes with
- *     the same launch plan (resident queries, prefs, precision, shape and
- *     buffers); a pass with another plan captures again.  With graph = 1
+ *     the same launch plan (counts and lengths of the resident queries,
+ *     model, tree, prior, prefs, precision, shape and buffers); a pass with
+ *     another plan captures again.  With graph = 1
  *     pp_stats holds the whole graph's device time in t_ml_ms and no
  *     per-phase or per-launch times.  0 (default) launches eagerly.
  * pp_launch_config_set returns PP_EINVAL, changing nothing, for a value out

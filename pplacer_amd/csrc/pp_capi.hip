@@ -445,7 +445,8 @@ int bucket_of(int M) { return M <= 0 ? 0 : (M - 1) / 64; }
 // Masked sites per worker lane in stage 2 for bucket b.  The FP64 kernels
 // hold one site's GLV rows per lane (two sites' rows spill at the 4 waves per
 // SIMD the kernels are built for); queries beyond 15 worker waves of one site
-// take two.  The FP32 kernels always hold two.
+// take two (one-rate models: with four rates the LDS account ends the classes
+// there, at 960 sites).  The FP32 kernels always hold two.
 int spl_for(bool fp64, int b) { return fp64 && b < 15 ? 1 : 2; }
 // one master wave + ceil(64 (b + 1) / (64 spl)) worker waves
 int block_for(int b, int spl) { return 64 * (1 + (b + spl) / spl); }
@@ -1084,16 +1085,11 @@ struct LaunchStream {
   ~LaunchStream() { c->cur = c->stream; }
 };
 
-// One placement pass over the resident queries, in chunks.  Stage 1 of every
-// chunk runs on its own stream into one of two score buffers, so it overlaps
-// stage 2 of the previous chunk; stage 2 (baseball, keep, refinement, -p,
-// finalize) runs chunk after chunk on the main stream; in the 4-state form a
-// phase's buckets can run concurrently on up to kBucketStreams streams (the
-// tails of their work queues overlap), joined before the next phase.
 // Short passes (kForkQueries): moves a chunk's queries of shorter masked-length
-// classes into the next longer class's launch while that holds at most two
-// rounds of the workgroups of its size that the device runs at once (4 waves
-// per SIMD).  Such launches last as long as their slowest query, and not all
+// classes into the next longer class's launch while its baseball then has at
+// most two rounds of the workgroups of its size that the device runs at once (4
+// waves per SIMD; the refinement and -p, with a job for each kept placement,
+// have more).  Such launches last as long as their slowest query, and not all
 // of them run at once (streams share hardware queues): one launch of 400 reads
 // with -p took 4.1 ms for the baseball phase where six over 4 streams took
 // 10.4, and the pass 17.9 -> 11.8 ms; 257 full-length reads 14.6 -> 11.7,
@@ -1122,7 +1118,13 @@ bool default_streams(const pp_launch_config &l, int f) {
   return l.pitch_streams[f] == kPitchStreams[f] && l.refine_streams[f] == kRefineStreams[f];
 }
 
-// form: whose streams of the launch shape the pass takes (0 or 1)
+// One placement pass over the resident queries, in chunks.  Stage 1 of every
+// chunk runs on its own stream into one of two score buffers, so it overlaps
+// stage 2 of the previous chunk; stage 2 (baseball, keep, refinement, -p,
+// finalize) runs chunk after chunk on the main stream; in the 4-state form a
+// phase's buckets can run concurrently on up to kBucketStreams streams (the
+// tails of their work queues overlap), joined before the next phase.  form:
+// whose streams of the launch shape the pass takes (0 or 1).
 int place_pass(pp_ctx *c, const pp_prefs *prefs, int precision, int form, pp_stats *stats) {
   CHECK(prefs, PP_EINVAL, "prefs is null");
   CHECK(precision == PP_FP64 || precision == PP_FP32, PP_EINVAL, "precision must be PP_FP64 or PP_FP32");
@@ -1177,8 +1179,7 @@ int place_pass(pp_ctx *c, const pp_prefs *prefs, int precision, int form, pp_sta
   const bool fp32 = precision == PP_FP32;
   const bool s2_fp32 = fp32 && stage2_fp32_ok(c);
   // Concurrent buckets (a short chunk's: kForkQueries), measured at 100,000
-  // queries: the FP32 form 323 -> 274
-  // ms per pass with 4 streams, 258 -> 251 ms with 8 for its baseball; the
+  // queries: the FP32 form 323 -> 274 ms per pass with 4 streams, 258 -> 251 ms with 8 for its baseball; the
   // refinement with 4 streams (FP64 364 -> 356 ms; with 50,000-query chunks
   // the FP32 form's 273-279 ms with 8 -> 267-270 ms with 4).  The FP64
   // baseball kernels stay on the main stream by default, so that each
