@@ -11,6 +11,10 @@ launch shape is:
   (the first pass of a new plan captures, the next ones replay; `pass_ms`
   keeps the best of its passes, so it times a replay).
 
+A form's default stream counts stand for the short-pass plan where chunks are
+short (include/pplacer_hip.h), so a search that starts from them times that
+plan first.
+
 Per-query results do not depend on the launch shape; only the time does, and
 it depends on the device, the tree and the query mix.  The search is
 coordinate-wise for one precision form: baseball streams, then refinement
